@@ -1,0 +1,78 @@
+"""The differentiable box's particle phase by bricks, at the sizes where its
+layout changes: sides shorter than a brick, ragged sides, bricks of 4 and of 8
+cells, every length of a particle block, boxes sorted by groups of bricks,
+moves longer than a cell, and particles outside the box.  FP64 against the
+PyTorch PIC and its autograd (bars of test_gpu_diff.py: 1e-12 forward, 1e-9
+adjoint)."""
+
+import numpy as np
+import pytest
+import torch
+
+import torch_pic as tp
+from runko_amd.diff import DiffBox
+from test_torch_pic import M, Q
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+
+
+def rel(a, b):
+    return float((a - b).norm() / b.norm().clamp_min(1e-300))
+
+
+def random_state(n, counts, seed):
+    g = torch.Generator(device=DEV)
+    g.manual_seed(seed)
+    E, B = (0.05 * torch.randn((3,) + n, generator=g, device=DEV, dtype=torch.float64) for _ in range(2))
+    hi = torch.tensor(n, device=DEV, dtype=torch.float64).view(3, 1)
+    x = torch.rand((3, sum(counts)), generator=g, device=DEV, dtype=torch.float64) * hi
+    u = 1.5 * torch.randn((3, sum(counts)), generator=g, device=DEV, dtype=torch.float64)
+    return E, B, x, u
+
+
+@pytest.mark.parametrize("n, counts, cfl", [
+    ((2, 3, 5), (40, 23), 0.45),            # sides shorter than a brick: windows wrap onto themselves
+    ((5, 9, 17), (700, 901), 0.45),         # ragged bricks of at most 4 cells, 7 blocks of 256 particles
+    ((6, 5, 9), (257, 1), 1.4),             # moves beyond the neighbouring cell
+    ((41, 18, 20), (70001, 70000), 0.45),   # blocks of 1024 particles
+    ((57, 66, 71), (530000, 530001), 0.45),  # bricks of at most 8 cells, blocks of 4096 particles
+    ((64, 64, 64), (2200000, 2100000), 0.45),  # blocks of 8192 particles
+    ((264, 256, 256), (60000, 60000), 0.45),  # sorted by groups of 2^3 bricks
+])
+def test_brick_layouts(n, counts, cfl):
+    s = random_state(n, counts, seed=sum(n))
+    box = DiffBox(n, Q, M, counts, cfl=cfl, dtype=torch.float64)
+    q = tp.per_particle(Q, counts, torch.float64, DEV)
+    qm = tp.per_particle([np.sign(a) / b for a, b in zip(Q, M)], counts, torch.float64, DEV)
+    leaves = tuple(t.clone().requires_grad_(True) for t in s)
+    ref = tp.step(*leaves, q, qm, cfl)
+    for name, a, b in zip("EBxu", box.step(s), ref):
+        assert rel(a, b.detach()) < 1e-12, name
+    g = torch.Generator(device=DEV)
+    g.manual_seed(3)
+    cot = tuple(torch.randn(t.shape, generator=g, device=DEV, dtype=torch.float64) for t in s)
+    grad = torch.autograd.grad(ref, leaves, grad_outputs=cot)
+    for name, a, b in zip("EBxu", box.step_adjoint(s, cot), grad):
+        assert rel(a, b) < 1e-9, name
+    assert box.error_count() == 0
+
+
+def test_particles_outside_the_box_pass_through():
+    n, counts = (9, 8, 7), (300, 300)
+    E, B, x, u = random_state(n, counts, seed=4)
+    inside = DiffBox(n, Q, M, counts, dtype=torch.float64).step((E, B, x, u))
+    x2, u2 = (torch.cat([v[:, :300], v[:, :1], v[:, 300:], v[:, -1:]], 1).contiguous() for v in (x, u))
+    x2[0, 300], x2[2, 601] = 14.0, float("nan")
+    box = DiffBox(n, Q, M, (301, 301), dtype=torch.float64)
+    out = box.step((E, B, x2, u2))
+    assert box.error_count() == 2
+    keep = [i for i in range(602) if i not in (300, 601)]
+    assert torch.equal(out[2][:, keep], inside[2]) and torch.equal(out[3][:, keep], inside[3])
+    assert rel(out[0], inside[0]) < 1e-12
+    assert torch.equal(out[2][:, 300], x2[:, 300]) and torch.equal(out[3][:, 601], u2[:, 601])
+    lam = tuple(torch.randn_like(t) for t in (E, B, x2, u2))
+    back = box.step_adjoint((E, B, x2, u2), lam)
+    for k in (300, 601):
+        assert torch.equal(back[2][:, k], lam[2][:, k]) and torch.equal(back[3][:, k], lam[3][:, k])
