@@ -234,3 +234,25 @@ def test_simulation_io_snapshots(tmp_path):
     assert "pspectra_0.bin" in names
     h = S.read_spectra_header(os.path.join(tmp_path, "pspectra_0.bin"))
     assert (h["nbins"], h["stride"]) == (200, 2)
+
+
+@pytest.mark.parametrize("n, stride, nbins, nspecies", [
+    ((12, 9, 10), 1, 60, 2),    # bricks of 6 x 1 x 5 cells, coarse cells inside one brick
+    ((12, 9, 10), 5, 60, 2),    # coarse cells and x bins shared by bricks, cells past the last one
+    ((8, 16, 16), 8, 5000, 2),  # more counters than a workgroup's LDS holds
+    ((16, 16, 16), 2, 128, 2),  # several bricks per workgroup (4^3 tiles)
+])
+def test_pack_counts_match_oracle(n, stride, nbins, nspecies):
+    nt = (4, 4, 4) if n == (16, 16, 16) else (2, 1, 2)
+    inputs, (conf, grid, sim) = random_grid(nt, n, seed=64, umax=2.0)
+    dims = [v for a in zip(nt, n) for v in a]
+    grid.world.call("rk_push_particles", -1)  # particles outside their bricks, and outside their tiles
+    pos, vel = tile_parts(grid, 2)
+    if stride <= min(n):
+        F = gpu_fields(grid).astype(F32)
+        got = S.MpiioFieldsWriter("unused", *dims, stride, nspecies).pack(grid).cpu().numpy()
+        ref = osnap.fields_pack([F[0], F[1], F[2]], [F[3], F[4], F[5]], [F[6], F[7], F[8]], pos, nt, n, stride, nspecies)
+        assert np.array_equal(got[9:], ref[9:])
+    got = S.MpiioSpectraWriter("unused", *dims, stride, nbins, 1e-2, 1e2, nspecies).pack(grid).cpu().numpy()
+    ref = osnap.spectra_pack([[p[0] for p in tp] for tp in pos], vel, nt, n, stride, nbins, 1e-2, 1e2, nspecies)
+    assert np.array_equal(got, ref)
