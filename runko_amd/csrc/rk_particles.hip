@@ -24,8 +24,8 @@
 // global memory.  Leavers are written to SoA migration records reserved with
 // one atomic per wave (ballot + popcount) and their slots are refilled from
 // the bin tail (swap-remove) so bins stay compact.  The fused step (k_fused)
-// does push, walls, classification, deposit and in-order compaction of a
-// brick in one workgroup.
+// does push, walls, classification, deposit and compaction of a brick in one
+// workgroup.
 #include "rk_internal.h"
 #include "rk_reflect.h"
 
@@ -310,6 +310,29 @@ __device__ inline float div_cfl(const Geo& g, float x)
   return FAST > 0 ? ieee_div(x, g.cfl) : x / g.cfl;
 }
 
+// x / cfl of a vector: one range check for its three components
+template<int FAST = 0>
+__device__ inline void div_cfl3(const Geo& g, const float x[3], float q[3])
+{
+  if constexpr(FAST > 0) {
+    const float hi = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fabsf(x[2]));
+    const float lo = fminf(fminf(fabsf(x[0]), fabsf(x[1])), fabsf(x[2]));
+    if(lo >= 0x1p-100f && hi <= 0x1p100f) {
+#pragma unroll
+      for(int c = 0; c < 3; ++c) {
+        const float t = x[c] * g.rcp_cfl;
+        q[c] = fmaf(fmaf(-t, g.cfl, x[c]), g.rcp_cfl, t);
+      }
+      return;
+    }
+#pragma unroll
+    for(int c = 0; c < 3; ++c) q[c] = ieee_div(x[c], g.cfl);
+  } else {
+#pragma unroll
+    for(int c = 0; c < 3; ++c) q[c] = div_cfl<FAST>(g, x[c]);
+  }
+}
+
 // Correctly rounded sqrt for 2^-60 <= x <= 2^60 from the hardware estimate
 // and a one-ulp residual test on each side, and c / s from the hardware
 // reciprocal (one Newton step) and one FMA remainder correction.  Used only
@@ -336,35 +359,37 @@ __device__ inline float div_near(float c, float s)
   return fmaf(e, r, q);
 }
 
-// cfl / sqrtf(X), X = cfl^2 + u.u (particle_boris.h:43,56)
+// cfl / sqrtf(X), X = cfl^2 + u.u (particle_boris.h:43,56): never below the
+// verified range's cfl^2, so only its upper end is checked
 template<int FAST = 0>
 __device__ inline float cfl_over_sqrt(const Geo& g, float X)
 {
-  if((FAST > 1 || (FAST == 0 && g.fast_sqrt)) && X >= g.cfl * g.cfl && X <= 0x1p60f)
+  if((FAST > 1 || (FAST == 0 && g.fast_sqrt)) && X <= 0x1p60f)
     return div_near(g.cfl, sqrt_near(X));
   return FAST > 1 ? ieee_div_sqrt(g.cfl, X) : g.cfl / sqrtf(X);
 }
 
-// c / t for c in {1, 2} and t = 1 + v.v (particle_boris.h:47, zigzag 1/sqrt)
+// 2 / t for t = 1 + v.v >= 1 (particle_boris.h:47)
 template<int FAST = 0>
 __device__ inline float two_over(const Geo& g, float t)
 {
-  if((FAST > 1 || (FAST == 0 && g.fast_sqrt)) && t >= 1.0f && t <= 0x1p60f) return div_near(2.0f, t);
+  if((FAST > 1 || (FAST == 0 && g.fast_sqrt)) && t <= 0x1p60f) return div_near(2.0f, t);
   return FAST > 1 ? ieee_div(2.0f, t) : 2.0f / t;
 }
 
-// 1 / t for t = 1 + b.b (particle_faraday.h)
+// 1 / t for t = 1 + b.b >= 1 (particle_faraday.h)
 template<int FAST = 0>
 __device__ inline float one_over(const Geo& g, float t)
 {
-  if((FAST > 1 || (FAST == 0 && g.fast_sqrt)) && t >= 1.0f && t <= 0x1p60f) return div_near(1.0f, t);
+  if((FAST > 1 || (FAST == 0 && g.fast_sqrt)) && t <= 0x1p60f) return div_near(1.0f, t);
   return FAST > 1 ? ieee_div(1.0f, t) : 1.0f / t;
 }
 
-template<int FAST = 0>
+// 1 / sqrt(t); ONE: t = 1 + v.v >= 1
+template<int FAST = 0, bool ONE = false>
 __device__ inline float inv_sqrt(const Geo& g, float t)
 {
-  if((FAST > 1 || (FAST == 0 && g.fast_sqrt)) && t >= 1.0f && t <= 0x1p60f) return div_near(1.0f, sqrt_near(t));
+  if((FAST > 1 || (FAST == 0 && g.fast_sqrt)) && (ONE || t >= 1.0f) && t <= 0x1p60f) return div_near(1.0f, sqrt_near(t));
   return FAST > 1 ? ieee_div_sqrt(1.0f, t) : 1.0f / sqrtf(t);
 }
 
@@ -382,9 +407,10 @@ __device__ inline void boris(const Geo& g, float qm, const float E[3], const flo
   }
   const float ginv = cfl_over_sqrt<FAST>(g, cfl * cfl + dot3(u0, u0));
   const float bfac = hq * ginv;
-  float B0[3];
+  float Bb[3], B0[3];
 #pragma unroll
-  for(int c = 0; c < 3; ++c) B0[c] = div_cfl<FAST>(g, B[c] * bfac);
+  for(int c = 0; c < 3; ++c) Bb[c] = B[c] * bfac;
+  div_cfl3<FAST>(g, Bb, B0);
   const float f = two_over<FAST>(g, 1.0f + dot3(B0, B0));
   float u1[3];
   u1[0] = (u0[0] + (u0[1] * B0[2] - u0[2] * B0[1])) * f;
@@ -394,8 +420,7 @@ __device__ inline void boris(const Geo& g, float qm, const float E[3], const flo
   u2[0] = (u0[0] + (u1[1] * B0[2] - u1[2] * B0[1])) + E0[0];
   u2[1] = (u0[1] + (-u1[0] * B0[2] + u1[2] * B0[0])) + E0[1];
   u2[2] = (u0[2] + (u1[0] * B0[1] - u1[1] * B0[0])) + E0[2];
-#pragma unroll
-  for(int c = 0; c < 3; ++c) vel[c] = div_cfl<FAST>(g, u2[c]);
+  div_cfl3<FAST>(g, u2, vel);
   const float ginv2 = cfl_over_sqrt<FAST>(g, cfl * cfl + dot3(u2, u2));
 #pragma unroll
   for(int c = 0; c < 3; ++c) pos[c] = pos[c] + (vel[c] * ginv2) * cfl;
@@ -417,7 +442,7 @@ template<int FAST = -1>
 __device__ inline Zig zigzag_setup(const Geo& g, const float x2[3], const float u[3], float charge, float cfl)
 {
   Zig z;
-  const float invgam = inv_sqrt<FAST>(g, 1.0f + dot3(u, u));
+  const float invgam = inv_sqrt<FAST, true>(g, 1.0f + dot3(u, u));
   const float s = cfl * invgam;
   float x1[3], fi1[3], fi2[3], xr[3], F1[3], F2[3], W1[3], W2[3];
 #pragma unroll
@@ -568,6 +593,12 @@ __device__ inline void stage_current(const CurWin& C, const double* ldsJ, float*
 // ---------------------------------------------------------------------------
 __device__ inline int lane_id() { return int(threadIdx.x) & 63; }
 
+// a float that is the same in every lane, in a scalar register
+__device__ inline float uniform_f(float v)
+{
+  return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)));
+}
+
 __device__ inline int64_t readfirstlane64(int64_t v)
 {
   const uint32_t lo = __builtin_amdgcn_readfirstlane(uint32_t(uint64_t(v)));
@@ -603,32 +634,6 @@ __device__ inline int block_rank(bool flag, int* wcnt, int& total)
   return off + __popcll(bal & lanemask_lt());
 }
 
-// Same scan with one barrier: the per-wave counts go to one of two buffers
-// that consecutive calls alternate (wcnt holds 2*NT/64 ints, par is flipped
-// here).  Call k+2 overwrites call k's buffer only after every wave passed
-// call k+1's barrier, i.e. after every read of call k.
-template<int NT>
-__device__ inline int block_rank1(bool flag, int* wcnt, int& par, int& total)
-{
-  constexpr int NW = NT / 64;
-  int* buf = wcnt + par * NW;
-  par ^= 1;
-  const uint64_t bal = __ballot(flag);
-  const int wid = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
-  if(lane_id() == 0) buf[wid] = __popcll(bal);
-  __syncthreads();
-  const int l = lane_id();
-  const int c = l < NW ? buf[l] : 0;
-  int x = c;
-  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);  // row_shr:1
-  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);  // row_shr:2
-  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);  // row_shr:4
-  if(NW > 8) x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);  // row_shr:8
-  const int off = __builtin_amdgcn_readlane(x - c, wid);
-  total = __builtin_amdgcn_readlane(x, NW - 1);
-  return off + __popcll(bal & lanemask_lt());
-}
-
 // reserve one slot per flagged lane in a counter with a single atomic per wave
 __device__ inline uint32_t wave_reserve(bool flag, uint32_t* counter)
 {
@@ -658,7 +663,7 @@ template<int NT = WG>
 struct CompactLdsT {
   uint32_t holes[MAX_HOLES];
   uint32_t tailbits[MAX_HOLES / 32];
-  int wcnt[2 * (NT / 64)];  // block_rank uses the first half, block_rank1 both
+  int wcnt[NT / 64];
   int nholes;
 };
 using CompactLds = CompactLdsT<WG>;
@@ -865,8 +870,7 @@ __device__ inline void faraday(const Geo& g, float qm, const float E[3], const f
   float u2[3];
 #pragma unroll
   for(int c = 0; c < 3; ++c) u2[c] = Wr[c] + er[c] * sc;
-#pragma unroll
-  for(int c = 0; c < 3; ++c) vel[c] = div_cfl<FAST>(g, u2[c]);
+  div_cfl3<FAST>(g, u2, vel);
   const float ginv2 = cfl_over_sqrt<FAST>(g, cfl * cfl + dot3p(u2, u2));
 #pragma unroll
   for(int c = 0; c < 3; ++c) pos[c] = pos[c] + vel[c] * ginv2 * cfl;
@@ -1250,7 +1254,6 @@ struct Shape {
   __device__ int D(int d) const { return b[d] + 3; }  // current nodes per axis
   __device__ int MV() const { return M(0) * M(1) * M(2); }
   __device__ int DV() const { return D(0) * D(1) * D(2); }
-  __device__ int div(int c, const Geo& g, int d) const { return BR > 0 ? c / BR : g.div_br(c, d); }
 };
 
 // node means of the brick window, one array per component (ex ey ez bx by bz)
@@ -1442,13 +1445,19 @@ __device__ inline void deposit_global(const Geo& g, const FieldPtrs& f, const Zi
   });
 }
 
-// fmodf(x, L) for L > 0; exact shortcut for |x| < 2L (Sterbenz: x -+ L is exact)
-__device__ inline float fmod_near(float x, float L)
+// fmodf(x, L) for L > 0 and |x| >= 2L (never taken by a particle that moved
+// less than the box): every subtraction is exact (r < 2y)
+__device__ inline float fmod_far(float x, float L)
 {
-  const float ax = fabsf(x);
-  if(ax < L) return x;
-  if(ax < 2.0f * L) return x - copysignf(L, x);
-  return fmodf(x, L);
+  float r = fabsf(x), y = L;
+  if(!(r < INFINITY)) return x - x;
+  while(y <= 0.5f * r) y *= 2.0f;
+  for(;;) {
+    if(r >= y) r -= y;
+    if(y <= L) break;
+    y *= 0.5f;
+  }
+  return copysignf(r, x);
 }
 
 // Element q of a bin array through a 32-bit byte offset from the bin's
@@ -1464,14 +1473,13 @@ __device__ inline T& at32(T* base, uint32_t q)
 // the brick's current window goes to its staging slot (no global atomics).
 constexpr int FWG = 512;  // 8 waves per brick
 
-// Per-brick constants of the tile-leaver path, indexed by axis and by the
-// step dv + 1 in {0, 1, 2} towards the destination tile (kept in LDS so they
-// occupy no scalar registers in the particle loop).
+// Per-brick constants of the tile-leaver path (kept in LDS so they occupy no
+// scalar registers in the particle loop): by axis and by the step dv + 1 in
+// {0, 1, 2} towards the destination tile, and the periodic box.
 struct NbrTab {
   float dorig[3][3];  // destination tile lattice origo: tile mins - 3
   int dtoffh[3][3];   // destination tile's world haloed offset
-  int off[3][3];      // destination tile-haloed node -> window index (unwrapped image)
-  float wlo[3], whi[3], wlen[3];  // periodic box
+  float box[3][3];    // low end, high end, length
 };
 
 // WALL: reflecting walls between the push and the classification
@@ -1529,19 +1537,45 @@ __device__ __attribute__((noinline)) void fused_deposit_global(float* J0, float*
   deposit_global(g, f, z, toffh, err);
 }
 
+// A wave's share of a bin's particles: whole 64-particle chunks, contiguous,
+// as even as they go.  Share i belongs to wave i, in odd species to wave
+// NW - 1 - i, so that one wave does not take the odd chunk of every species.
+struct Share {
+  int t0, t1;
+};
+
+template<int NW>
+__device__ inline int share_wave(int s, int i) { return s & 1 ? NW - 1 - i : i; }
+
+template<int NW>
+__device__ inline Share wave_share(int count, int s, int wave)
+{
+  const int i = share_wave<NW>(s, wave);  // (its own inverse)
+  const int chunks = (count + 63) / 64, q = chunks / NW, r = chunks % NW;
+  const int c0 = i * q + min(i, r), c1 = c0 + q + (i < r ? 1 : 0);
+  return Share {min(c0 * 64, count), min(c1 * 64, count)};
+}
+
 template<int BR, int FAST, int WALL, int PUSHER, int WGS>
 __device__ __forceinline__ void fused_brick(const Geo& g, const SpParams& sp, const FieldPtrs& f, const MigPtrs& m,
                                             const MigPtrs* mtab, int b, uint32_t* counters, float* jstage,
                                             int64_t jstage_stride, const WallSet& walls, float* Jc0, float* Jc1,
-                                            float* Jc2, double* lds_dyn, int* wcnt, NbrTab& NT)
+                                            float* Jc2, double* lds_dyn, uint32_t (*left)[WGS / 64], uint32_t* nrec, NbrTab& NT)
 {
   const Shape<BR> S(g);
-  const Brick Bk = brick_of(g, b);
+  Brick Bk = brick_of(g, b);
+#pragma unroll
+  for(int d = 0; d < 3; ++d) {
+    Bk.tmin[d] = uniform_f(Bk.tmin[d]);
+    Bk.tmax[d] = uniform_f(Bk.tmax[d]);
+    Bk.origo[d] = uniform_f(Bk.origo[d]);
+  }
   uint64_t* ldsJ = reinterpret_cast<uint64_t*>(lds_dyn);
   float* ldsM = reinterpret_cast<float*>(lds_dyn + 3 * S.DV());
   for(int q = int(threadIdx.x); q < 3 * S.DV(); q += WGS) ldsJ[q] = 0;
   const bool any = bin_total(sp, b) != 0;
   if(any) stage_means6<BR, WGS>(g, f, S, Bk.c0, ldsM);
+  if(threadIdx.x == 0) *nrec = 0;
   __syncthreads();
   // window index of a particle's cell: tile-haloed cell - 3 - lb*br (means),
   // tile-haloed node - 2 - lb*br (current)
@@ -1551,25 +1585,42 @@ __device__ __forceinline__ void fused_brick(const Geo& g, const SpParams& sp, co
     moff[d] = -HALO - Bk.lb[d] * S.b[d];
     coff[d] = moff[d] + 1;
   }
+  // the brick's faces, relative to the tile lattice origo
+  float blo[3], bhi[3];
+#pragma unroll
+  for(int d = 0; d < 3; ++d) {
+    const float lo = float(HALO + Bk.lb[d] * S.b[d]);
+    blo[d] = uniform_f(lo);
+    bhi[d] = uniform_f(Bk.lb[d] == g.nb[d] - 1 ? INFINITY : lo + float(S.b[d]));
+  }
   if(threadIdx.x < 9) {
     const int d = int(threadIdx.x) / 3, k = int(threadIdx.x) % 3;
     int tc = Bk.tc[d] + k - 1;
     tc = tc < 0 ? tc + g.nt[d] : (tc >= g.nt[d] ? tc - g.nt[d] : tc);
     NT.dorig[d][k] = g.tile_min(tc, d) - 3.0f;
     NT.dtoffh[d][k] = tc * g.n[d];
-    // the destination's nodes sit next to this tile in the unwrapped frame:
-    // the image nearest to this brick
-    NT.off[d][k] = (k - 1) * g.n[d] - HALO + 1 - Bk.lb[d] * S.b[d];
     if(k == 0) {
-      NT.wlo[d] = g.wmin[d];
-      NT.whi[d] = g.wmax[d];
-      NT.wlen[d] = g.wmax[d] - g.wmin[d];
+      NT.box[d][0] = g.wmin[d];
+      NT.box[d][1] = g.wmax[d];
+      NT.box[d][2] = g.wmax[d] - g.wmin[d];
     }
   }
   __syncthreads();
   // walls in this brick's tile (uniform over the block)
   const unsigned wmask = WALL ? walls_in_tile(walls, Bk.tmin[0], Bk.tmax[0], g.cfl) : 0u;
-  int nrec = 0;  // records in this brick's mailbox (uniform over the block)
+  // Each wave takes a contiguous share of a species' 64-particle chunks and
+  // compacts it in place: the survivors of a chunk go to the running offset wr
+  // (at most the chunk's first slot, and every lane holds its particle in
+  // registers), so no barrier and no block-wide scan runs in the particle
+  // loop, and the waves drift apart: the gathers and current adds of some
+  // overlap the arithmetic of others.  The gaps at the ends of the shares are
+  // closed afterwards (below).  VALU issue bounds the loop (88 % busy at 256^3,
+  // 32 particles per cell).  Against a block-wide scan of every 512-particle
+  // chunk with a barrier each: 256^3 12.56 -> 11.98 ms, 64^3 128 -> 120 us,
+  // with the classification by brick faces and the shorter exact forms.
+  constexpr int NW = WGS / 64;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+  const int lane = lane_id();
   for(int s = 0; any && s < sp.nsp; ++s) {
     // bin start and count are uniform: keep them (and the bin's array bases)
     // scalar so particle addresses are a 32-bit lane offset from a scalar base
@@ -1579,7 +1630,7 @@ __device__ __forceinline__ void fused_brick(const Geo& g, const SpParams& sp, co
     const float qm = sp.qm[s];
     const float charge = sp.charge[s];
     // the deposit's charge in the window's fixed-point unit (exact: a power of two)
-    const float qscaled = charge * float(g.jscale), jinv_f = float(g.jinv);
+    const float qscaled = uniform_f(charge * float(g.jscale));
     float* const P0 = sp.pos[s][0] + start;
     float* const P1 = sp.pos[s][1] + start;
     float* const P2 = sp.pos[s][2] + start;
@@ -1587,18 +1638,14 @@ __device__ __forceinline__ void fused_brick(const Geo& g, const SpParams& sp, co
     float* const U1 = sp.vel[s][1] + start;
     float* const U2 = sp.vel[s][2] + start;
     uint64_t* const ID = sp.id[s] + start;
-    // In-order compaction: the survivors of every chunk are written at the
-    // running offset wr (wr <= the chunk's first slot, and every lane holds
-    // its particle in registers before the scan's barrier), so the bin ends
-    // compact with whole-line writes and no separate compaction pass.
-    int wr = 0;
-    int par = 0;
-    // the next chunk's particles are loaded one iteration ahead, so their
-    // latency overlaps this chunk's arithmetic
+    const Share sh = wave_share<NW>(count, s, wave);
+    int wr = sh.t0;
+    // the next chunk's particles are loaded during this chunk's deposit (from
+    // its start they would hold registers through the push: spills)
     float npos[3] = {0.0f, 0.0f, 0.0f}, nvel[3] = {0.0f, 0.0f, 0.0f};
     uint64_t nid = 0;
-    if(int(threadIdx.x) < count) {
-      const uint32_t q0 = threadIdx.x;
+    if(sh.t0 + lane < sh.t1) {
+      const uint32_t q0 = uint32_t(sh.t0 + lane);
       npos[0] = at32(P0, q0);
       npos[1] = at32(P1, q0);
       npos[2] = at32(P2, q0);
@@ -1607,23 +1654,13 @@ __device__ __forceinline__ void fused_brick(const Geo& g, const SpParams& sp, co
       nvel[2] = at32(U2, q0);
       nid = at32(ID, q0);
     }
-    for(int base = 0; base < count; base += WGS) {
-      const int t = base + int(threadIdx.x);
+    for(int base = sh.t0; base < sh.t1; base += 64) {
+      const int t = base + lane;
       bool lv0 = false, lv1 = false, dead = false;
       float pos[3] = {npos[0], npos[1], npos[2]}, vel[3] = {nvel[0], nvel[1], nvel[2]};
       const uint64_t id = nid;
       int dir = 13;
-      if(t + WGS < count) {
-        const uint32_t qn = uint32_t(t + WGS);
-        npos[0] = at32(P0, qn);
-        npos[1] = at32(P1, qn);
-        npos[2] = at32(P2, qn);
-        nvel[0] = at32(U0, qn);
-        nvel[1] = at32(U1, qn);
-        nvel[2] = at32(U2, qn);
-        nid = at32(ID, qn);
-      }
-      if(t < count) {
+      if(t < sh.t1) {
         float pr[3], dd[3];
         int ci[3];
 #pragma unroll
@@ -1653,81 +1690,97 @@ __device__ __forceinline__ void fused_brick(const Geo& g, const SpParams& sp, co
                                    &counters[C_STENCIL]);
         }
       }
-      if(t < count && !dead) {
-        // classification against the tile (pack_outgoing) and the brick
-        dir = tile_dir(pos, Bk.tmin, Bk.tmax);
+      if(t + 64 < sh.t1) {
+        const uint32_t qn = uint32_t(t + 64);
+        npos[0] = at32(P0, qn);
+        npos[1] = at32(P1, qn);
+        npos[2] = at32(P2, qn);
+        nvel[0] = at32(U0, qn);
+        nvel[1] = at32(U1, qn);
+        nvel[2] = at32(U2, qn);
+        nid = at32(ID, qn);
+      }
+      if(t < sh.t1 && !dead) {
+        // classification against the tile (pack_outgoing) and the brick: the
+        // brick of the particle's cell, floor(x2) - 3 clamped to the tile, is
+        // this one when x2 lies between the brick's faces (a face on the
+        // tile's boundary bounds nothing)
         float x2[3];
-        int off[3], dtoffh[3];
-        if(dir != 13) {
-          lv0 = true;
-          const int k3[3] = {dir / 9, (dir / 3) % 3, dir % 3};
+        int off[3];
+        bool inside = true;
+#pragma unroll
+        for(int d = 0; d < 3; ++d) {
+          x2[d] = pos[d] - Bk.origo[d];
+          off[d] = coff[d];
+          inside = inside && (Bk.lb[d] == 0 || x2[d] >= blo[d]) && !(x2[d] >= bhi[d]);
+          lv0 = lv0 || pos[d] < Bk.tmin[d] || pos[d] >= Bk.tmax[d];
+        }
+        lv1 = !lv0 && !inside;
+        if(lv0) {
+          int k3[3];
 #pragma unroll
           for(int d = 0; d < 3; ++d) {
-            // every coordinate wrapped by the global box, particle.h:523-549
-            const float pw = (pos[d] < 0 ? NT.whi[d] : NT.wlo[d]) + fmod_near(pos[d], NT.wlen[d]);
-            x2[d] = pw - NT.dorig[d][k3[d]];
-            dtoffh[d] = NT.dtoffh[d][k3[d]];
-            off[d] = NT.off[d][k3[d]];
+            k3[d] = pos[d] < Bk.tmin[d] ? 0 : (pos[d] >= Bk.tmax[d] ? 2 : 1);
+            // every coordinate wrapped by the global box, particle.h:523-549:
+            // (x < 0 ? max : min) + fmod(x, L), exact shortcuts for |x| < 2L (Sterbenz)
+            const float L = NT.box[d][2], ax = fabsf(pos[d]);
+            float f = ax < L ? pos[d] : pos[d] - copysignf(L, pos[d]);
+            if(ax >= 2.0f * L) f = fmod_far(pos[d], L);
+            x2[d] = ((pos[d] < 0 ? NT.box[d][1] : NT.box[d][0]) + f) - NT.dorig[d][k3[d]];
+            // the destination's nodes sit next to this tile in the unwrapped
+            // frame: the image nearest to this brick
+            off[d] += (k3[d] - 1) * g.n[d];
           }
-        } else {
-          int lb[3];
-#pragma unroll
-          for(int d = 0; d < 3; ++d) {
-            x2[d] = pos[d] - Bk.origo[d];
-            const int c = min(max(int(floorf(x2[d])) - HALO, 0), g.n[d] - 1);
-            lb[d] = BR > 0 ? int(uint32_t(c) / uint32_t(BR)) : S.div(c, g, d);
-            off[d] = coff[d];
-            dtoffh[d] = Bk.toffh[d];
-          }
-          lv1 = lb[0] != Bk.lb[0] || lb[1] != Bk.lb[1] || lb[2] != Bk.lb[2];
+          dir = 9 * k3[0] + 3 * k3[1] + k3[2];
         }
         // zigzag deposit in the frame of the tile that owns the particle after migration
         const Zig z = zigzag_setup<FAST>(g, x2, vel, qscaled, g.cfl);
         if(!deposit_win(S, ldsJ, z, off))
-          fused_deposit_global(f.J[0], f.J[1], f.J[2], g.L[0], g.L[1], g.L[2], unscaled(z, jinv_f), dtoffh[0],
-                               dtoffh[1], dtoffh[2], &counters[C_STENCIL]);
+          fused_deposit_global(f.J[0], f.J[1], f.J[2], g.L[0], g.L[1], g.L[2], unscaled(z, float(g.jinv)),
+                               NT.dtoffh[0][dir / 9], NT.dtoffh[1][dir / 3 % 3], NT.dtoffh[2][dir % 3],
+                               &counters[C_STENCIL]);
       }
-      // leavers take consecutive slots of this brick's mailbox (rank from a
-      // block scan: no global atomics); past its capacity they spill into
-      // the shared record sets
+      // leavers take consecutive slots of this brick's mailbox (the wave's
+      // reserved with one LDS atomic); past its capacity they spill into the
+      // shared record sets
+      // (a fence for the scheduler: without it the loop's registers spill)
+      __builtin_amdgcn_wave_barrier();
       const bool hole = lv0 || lv1;
-      int tot;
-      const int r = block_rank1<WGS>(hole, wcnt, par, tot);
-      const int64_t local = int64_t(nrec) + r;
-      bool spill = false, kept = false;
-      uint32_t slot0 = 0, slot1 = 0;
-      if(int64_t(nrec) + tot > m.per_brick) {
-        // uniform: this chunk fills the mailbox
-        spill = hole && local >= m.per_brick;
-        slot0 = wave_reserve(spill && lv0, &counters[C_MIG0]);
-        slot1 = wave_reserve(spill && lv1, &counters[C_MIG1]);
-        if(spill && ((lv0 && int64_t(slot0) >= mtab->cap[0]) || (lv1 && int64_t(slot1) >= mtab->cap[1]))) {
-          // no room anywhere: the particle stays in this bin (pushed and
-          // deposited); it is classified again next step
-          kept = true;
-          atomicAdd(&counters[C_MIGLOST], 1u);
+      const uint64_t holes = __ballot(hole);
+      bool kept = false;
+      if(holes != 0) {
+        const int tot = __popcll(holes);
+        int first = 0;
+        if(lane == 0) first = int(atomicAdd(nrec, uint32_t(tot)));
+        first = __builtin_amdgcn_readfirstlane(first);
+        const int64_t local = int64_t(first) + __popcll(holes & lanemask_lt());
+        bool spill = false;
+        uint32_t slot0 = 0, slot1 = 0;
+        if(int64_t(first) + tot > m.per_brick) {
+          // uniform over the wave: this chunk fills the mailbox
+          spill = hole && local >= m.per_brick;
+          slot0 = wave_reserve(spill && lv0, &counters[C_MIG0]);
+          slot1 = wave_reserve(spill && lv1, &counters[C_MIG1]);
+          if(spill && ((lv0 && int64_t(slot0) >= mtab->cap[0]) || (lv1 && int64_t(slot1) >= mtab->cap[1]))) {
+            // no room anywhere: the particle stays in this bin (pushed and
+            // deposited); it is classified again next step
+            kept = true;
+            atomicAdd(&counters[C_MIGLOST], 1u);
+          }
+        }
+        if(hole && !kept) {
+          // records keep the unwrapped position; the append applies the wrap
+          const uint32_t meta = lv0 ? meta_pack(s, 0, dir, uint32_t(b)) : meta_pack(s, 1, 13, uint32_t(b));
+          if(!spill) write_record(m, 2, uint32_t(int64_t(b) * m.per_brick + local), pos, vel, id, meta);
+          else
+            fused_spill_record(mtab, lv0 ? 0 : 1, lv0 ? slot0 : slot1, pos[0], pos[1], pos[2], vel[0], vel[1], vel[2],
+                               id, meta);
         }
       }
-      const bool stays = t < count && !dead && (!hole || kept);
-      // survivor's slot: wr + lanes before it in the chunk - leavers before
-      // it that departed (r counts all leavers, rk the kept ones)
-      int kept_tot = 0;
-      int rk = 0;
-      if(int64_t(nrec) + tot > m.per_brick) rk = block_rank1<WGS>(hole && kept, wcnt, par, kept_tot);
-      // parked particles before this lane (they are not leavers)
-      int dead_tot = 0, rd = 0;
-      if(WALL && wmask) rd = block_rank1<WGS>(dead, wcnt, par, dead_tot);
-      const int dst = wr + int(threadIdx.x) - (r - rk) - rd;
-      if(t < count && hole && !kept) {
-        // records keep the unwrapped position; the append applies the wrap
-        const uint32_t meta = lv0 ? meta_pack(s, 0, dir, uint32_t(b)) : meta_pack(s, 1, 13, uint32_t(b));
-        if(!spill) write_record(m, 2, uint32_t(int64_t(b) * m.per_brick + local), pos, vel, id, meta);
-        else
-          fused_spill_record(mtab, lv0 ? 0 : 1, lv0 ? slot0 : slot1, pos[0], pos[1], pos[2], vel[0], vel[1], vel[2], id,
-                             meta);
-      }
+      const bool stays = t < sh.t1 && !dead && (!hole || kept);
+      const uint64_t staying = __ballot(stays);
       if(stays) {
-        const uint32_t d = uint32_t(dst);
+        const uint32_t d = uint32_t(wr + __popcll(staying & lanemask_lt()));
         at32(P0, d) = pos[0];
         at32(P1, d) = pos[1];
         at32(P2, d) = pos[2];
@@ -1736,15 +1789,47 @@ __device__ __forceinline__ void fused_brick(const Geo& g, const SpParams& sp, co
         at32(U2, d) = vel[2];
         if(d != uint32_t(t)) at32(ID, d) = id;
       }
-      wr += min(WGS, count - base) - (tot - kept_tot) - dead_tot;
-      nrec += (int64_t(nrec) + tot <= m.per_brick) ? tot : int(m.per_brick - nrec);
+      wr += __popcll(staying);
     }
-    __syncthreads();
-    if(threadIdx.x == 0) sp.count[s][b] = uint32_t(wr);
-    __syncthreads();
+    if(lane == 0) left[s][wave] = uint32_t(wr - sh.t0);
   }
-  if(threadIdx.x == 0) m.mcount[b] = uint32_t(nrec);
   __syncthreads();
+  if(threadIdx.x == 0) m.mcount[b] = uint32_t(min(int64_t(*nrec), m.per_brick));
+  // Close the gaps: the bin ends compact in [0, total).  The slots of
+  // [0, total) behind a share's survivors take, in order, the survivors that
+  // lie at total and beyond.
+  for(int s = 0; any && s < sp.nsp; ++s) {
+    const int count = __builtin_amdgcn_readfirstlane(int(sp.count[s][b]));
+    if(count == 0) continue;
+    int total = 0;
+#pragma unroll 1
+    for(int w = 0; w < NW; ++w) total += int(left[s][w]);
+    const int64_t start = readfirstlane64(sp.start[s][b]);
+    // the k-th hole and the k-th stray survivor (shares in the order of their slots)
+    for(int k = int(threadIdx.x);; k += WGS) {
+      int hole = -1, stray = -1, nh = 0, ns = 0;
+#pragma unroll 1
+      for(int i = 0; i < NW; ++i) {
+        const int w = share_wave<NW>(s, i);
+        const Share sh = wave_share<NW>(count, s, w);
+        const int end = sh.t0 + int(left[s][w]);
+        const int h = max(0, min(sh.t1, total) - end), st0 = max(sh.t0, total), st = max(0, end - st0);
+        if(k >= nh && k < nh + h) hole = end + (k - nh);
+        if(k >= ns && k < ns + st) stray = st0 + (k - ns);
+        nh += h;
+        ns += st;
+      }
+      if(hole < 0) break;  // past the last hole
+#pragma unroll
+      for(int d = 0; d < 3; ++d) {
+        sp.pos[s][d][start + hole] = sp.pos[s][d][start + stray];
+        sp.vel[s][d][start + hole] = sp.vel[s][d][start + stray];
+      }
+      sp.id[s][start + hole] = sp.id[s][start + stray];
+    }
+    __syncthreads();  // every thread has read the old count
+    if(threadIdx.x == 0) sp.count[s][b] = uint32_t(total);
+  }
   const int V3 = 3 * S.DV();
   float* stage = jstage + int64_t(b) * jstage_stride;
   for(int q = int(threadIdx.x); q < V3; q += WGS) stage[q] = float(double(int64_t(ldsJ[q])) * g.jinv);
@@ -1763,7 +1848,8 @@ __global__ void __launch_bounds__(WGS) __attribute__((amdgpu_waves_per_eu(4)))
           float* Jc2)
 {
   extern __shared__ double lds_dyn[];
-  __shared__ int wcnt[2 * (WGS / 64)];
+  __shared__ uint32_t left[RK_MAX_SPECIES][WGS / 64];  // survivors of every share
+  __shared__ uint32_t nrec;                            // leavers of the brick
   __shared__ NbrTab NT;
   // the walls (from the launch arguments, or from device memory when wdev
   // is given: walls that move on the device), staged in LDS
@@ -1778,7 +1864,7 @@ __global__ void __launch_bounds__(WGS) __attribute__((amdgpu_waves_per_eu(4)))
     const int b = xcd_brick(int(blockIdx.x), span);
     if(b >= nbins) return;
     fused_brick<BR, FAST, WALL, PUSHER, WGS>(g, sp, f, m, mtab, b, counters, jstage, jstage_stride, sw, Jc0, Jc1, Jc2,
-                                        lds_dyn, wcnt, NT);
+                                        lds_dyn, left, &nrec, NT);
   } else {
     __shared__ int next;
     const int x = int(blockIdx.x) % 8;
@@ -1789,7 +1875,7 @@ __global__ void __launch_bounds__(WGS) __attribute__((amdgpu_waves_per_eu(4)))
       __syncthreads();
       if(b >= nbins) break;  // uniform: every later pop of this queue is past the end too
       fused_brick<BR, FAST, WALL, PUSHER, WGS>(g, sp, f, m, mtab, b, counters, jstage, jstage_stride, sw, Jc0, Jc1,
-                                          Jc2, lds_dyn, wcnt, NT);
+                                          Jc2, lds_dyn, left, &nrec, NT);
       __syncthreads();  // the brick's LDS is read out before the next brick fills it
     }
   }
@@ -2293,17 +2379,18 @@ int launch_fused(rk_world* w, hipStream_t s, const WallSet* walls, const rk_refl
     return RK_EINVAL;
   }
   if(g.pusher != 0) {
-    // Higuera-Cary or Faraday, 8^3 bricks or the generic shape; on 8^3 bricks
-    // with both fast forms verified, the pusher, the deposit and the
-    // classification take the verified sqrt/rcp forms (the IEEE results),
-    // otherwise the IEEE operations
+    // Higuera-Cary or Faraday, 8^3 bricks or the generic shape; with both fast
+    // forms verified, the pusher, the deposit and the classification take the
+    // verified sqrt/rcp forms (the IEEE results), otherwise the IEEE operations
     const bool hc = g.pusher == 1;
     if(ws.n > 0) {
       if(cube8 && lvl == 2) hc ? go(k_fused<8, 2, 1, 1>) : go(k_fused<8, 2, 1, 2>);
       else if(cube8) hc ? go(k_fused<8, -1, 1, 1>) : go(k_fused<8, -1, 1, 2>);
+      else if(lvl == 2) hc ? go(k_fused<0, 2, 1, 1>) : go(k_fused<0, 2, 1, 2>);
       else hc ? go(k_fused<0, -1, 1, 1>) : go(k_fused<0, -1, 1, 2>);
     } else if(cube8 && lvl == 2) hc ? go(k_fused<8, 2, 0, 1>) : go(k_fused<8, 2, 0, 2>);
     else if(cube8) hc ? go(k_fused<8, -1, 0, 1>) : go(k_fused<8, -1, 0, 2>);
+    else if(lvl == 2) hc ? go(k_fused<0, 2, 0, 1>) : go(k_fused<0, 2, 0, 2>);
     else hc ? go(k_fused<0, -1, 0, 1>) : go(k_fused<0, -1, 0, 2>);
   } else if(w->fused_wg == 256 && cube8 && !w->fused_queue) {
     auto go256 = [&](auto kern) {
@@ -2340,10 +2427,10 @@ int launch_fused(rk_world* w, hipStream_t s, const WallSet* walls, const rk_refl
   } else if(ws.n > 0) {
     if(cube8) lvl == 2 ? go(k_fused<8, 2, 1>) : (lvl == 1 ? go(k_fused<8, 1, 1>) : go(k_fused<8, -1, 1>));
     else if(cube4) lvl == 2 ? go(k_fused<4, 2, 1>) : (lvl == 1 ? go(k_fused<4, 1, 1>) : go(k_fused<4, -1, 1>));
-    else go(k_fused<0, 0, 1>);
+    else lvl == 2 ? go(k_fused<0, 2, 1>) : go(k_fused<0, 0, 1>);
   } else if(cube8) lvl == 2 ? go(k_fused<8, 2>) : (lvl == 1 ? go(k_fused<8, 1>) : go(k_fused<8, -1>));
   else if(cube4) lvl == 2 ? go(k_fused<4, 2>) : (lvl == 1 ? go(k_fused<4, 1>) : go(k_fused<4, -1>));
-  else go(k_fused<0, 0>);
+  else lvl == 2 ? go(k_fused<0, 2>) : go(k_fused<0, 0>);
   RK_HIP(hipGetLastError());
   return RK_OK;
 }
