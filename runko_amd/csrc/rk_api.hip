@@ -656,15 +656,12 @@ int fused_step(rk_world* w, const rk_reflector_wall* walls, int32_t n_walls, boo
     if(int rc = launch_fused(w, s, &ws, device_walls ? w->walls_dev : nullptr)) return rc;
   }
   {
-    ProfScope ps(w, 2, s);
-    if(int rc = launch_current_gather(w, s)) return rc;
-    if(int rc = apply_corrections(w, -1, s)) return rc;
-    if(device_walls && ws.n > 0)
-      if(int rc = add_corrections_world(w, s)) return rc;
+    ProfScope ps(w, 4, s);
+    if(int rc = launch_fused_tail(w, s)) return rc;
   }
-  ProfScope ps(w, 4, s);
-  if(int rc = launch_append_mailbox(w, s)) return rc;
-  return launch_append_records(w, s);
+  ProfScope ps(w, 2, s);
+  if(int rc = apply_corrections(w, -1, s)) return rc;
+  return device_walls && ws.n > 0 ? add_corrections_world(w, s) : RK_OK;
 }
 }  // namespace
 

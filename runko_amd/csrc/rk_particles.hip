@@ -1116,23 +1116,23 @@ __global__ void __launch_bounds__(WG)
   }
 }
 
-// Append the records of sets 0 and 1 (blockIdx.y is the set), then clear
-// both record counters: every workgroup reads its set's count before it
-// signs off on C_APPDONE, and the last workgroup to sign off clears C_MIG0,
-// C_MIG1 and C_APPDONE, so the counters are zero for the next step without
-// separate launches.
-__global__ void __launch_bounds__(WG)
-  k_append_records(Geo g, SpParams sp, MigPtrs m, uint32_t* counters, uint32_t* ovf, int64_t ovf_cap)
+// Append the records of sets 0 and 1, then clear both record counters: the
+// blocks of a launch that do this (`blocks` of them, the first half for set 0)
+// read their set's count before they sign off on C_APPDONE, and the last one
+// to sign off clears C_MIG0, C_MIG1 and C_APPDONE, so the counters are zero
+// for the next step without separate launches.
+__device__ inline void append_records(const Geo& g, const SpParams& sp, const MigPtrs& m, int blk, int blocks,
+                                      uint32_t* counters, uint32_t* ovf, int64_t ovf_cap)
 {
-  const int set = int(blockIdx.y);
+  const int per = blocks / 2, set = blk / per;
   const int n = int(min(int64_t(counters[set == 0 ? C_MIG0 : C_MIG1]), m.cap[set]));
-  for(int e = int(blockIdx.x * blockDim.x + threadIdx.x); e < n; e += int(gridDim.x * blockDim.x))
+  for(int e = (blk % per) * WG + int(threadIdx.x); e < n; e += per * WG)
     append_record(g, sp, m, set, uint32_t(e), counters, ovf, ovf_cap);
   __syncthreads();
   if(threadIdx.x == 0) {
     __threadfence();
     const uint32_t done = atomicAdd(&counters[C_APPDONE], 1u);
-    if(done == gridDim.x * gridDim.y - 1) {
+    if(done == uint32_t(blocks - 1)) {
       counters[C_MIG0] = 0;
       counters[C_MIG1] = 0;
       counters[C_APPDONE] = 0;
@@ -1149,86 +1149,79 @@ __device__ inline int global_brick(const Geo& g, int b, int d)
   return tc[d] * g.nb[d] + lb[d];
 }
 
-// Append every brick's mailbox, then empty it.  Records of one brick go to
-// the brick itself or its 26 periodic neighbours: per chunk of WG records
-// the slots of each (species, neighbour) pair are ranked with LDS atomics and
-// reserved with one global atomic per pair.
-__global__ void __launch_bounds__(WG)
-  k_append_mailbox(Geo g, SpParams sp, MigPtrs m, int nbins, uint32_t* counters, uint32_t* ovf, int64_t ovf_cap, int span)
+// Append brick b's mailbox, then empty it (a workgroup of WG threads).  Records
+// of one brick go to the brick itself or its 26 periodic neighbours: per chunk
+// of WG records the slots of each (species, neighbour) pair are ranked with LDS
+// atomics and reserved with one global atomic per pair.
+__device__ inline void append_mailbox(const Geo& g, const SpParams& sp, const MigPtrs& m, int b, uint32_t* counters,
+                                      uint32_t* ovf, int64_t ovf_cap)
 {
   constexpr int NK = RK_MAX_SPECIES * 27;
   __shared__ uint32_t cnt[NK];
   __shared__ uint32_t kbase[NK];
   __shared__ int kdb[NK];
-  // one block per brick, with the fused step's XCD-aware brick map: a brick's
-  // neighbours mostly run on the same XCD, so the appends to one destination
-  // bin's tail mostly go through one L2
-  {
-    const int b = xcd_brick(int(blockIdx.x), span);
-    if(b >= nbins) return;  // uniform over the block
-    const int n = int(m.mcount[b]);
-    if(n == 0) return;  // uniform over the block
-    const uint32_t base = uint32_t(int64_t(b) * m.per_brick);
-    int gsrc[3];
+  const int n = int(m.mcount[b]);
+  if(n == 0) return;  // uniform over the block
+  const uint32_t base = uint32_t(int64_t(b) * m.per_brick);
+  int gsrc[3];
 #pragma unroll
-    for(int d = 0; d < 3; ++d) gsrc[d] = global_brick(g, b, d);
-    for(int c0 = 0; c0 < n; c0 += WG) {
-      for(int k = int(threadIdx.x); k < NK; k += WG) cnt[k] = 0;
-      __syncthreads();
-      const int e = c0 + int(threadIdx.x);
-      RecordDest R;
-      int key = -1;
-      uint32_t rank = 0;
-      // the record's payload is loaded with its destination, so its latency
-      // overlaps the ranking and the reservation
-      float rv[3] = {0.0f, 0.0f, 0.0f};
-      uint64_t rid = 0;
-      if(e < n) {
-        const uint32_t r = base + uint32_t(e);
+  for(int d = 0; d < 3; ++d) gsrc[d] = global_brick(g, b, d);
+  for(int c0 = 0; c0 < n; c0 += WG) {
+    for(int k = int(threadIdx.x); k < NK; k += WG) cnt[k] = 0;
+    __syncthreads();
+    const int e = c0 + int(threadIdx.x);
+    RecordDest R;
+    int key = -1;
+    uint32_t rank = 0;
+    // the record's payload is loaded with its destination, so its latency
+    // overlaps the ranking and the reservation
+    float rv[3] = {0.0f, 0.0f, 0.0f};
+    uint64_t rid = 0;
+    if(e < n) {
+      const uint32_t r = base + uint32_t(e);
 #pragma unroll
-        for(int d = 0; d < 3; ++d) rv[d] = m.vel[2][d][r];
-        rid = m.id[2][r];
-        R = record_dest(g, m, 2, r);
-        int off = 0;
-        bool near = true;
+      for(int d = 0; d < 3; ++d) rv[d] = m.vel[2][d][r];
+      rid = m.id[2][r];
+      R = record_dest(g, m, 2, r);
+      int off = 0;
+      bool near = true;
+#pragma unroll
+      for(int d = 0; d < 3; ++d) {
+        const int NB = g.nt[d] * g.nb[d];
+        int df = global_brick(g, R.db, d) - gsrc[d];
+        df = df < 0 ? df + NB : df;
+        const int o = df == 0 ? 0 : (df == 1 ? 1 : (df == NB - 1 ? -1 : 2));
+        near = near && o != 2;
+        off = off * 3 + (o + 1);
+      }
+      if(near) {
+        key = R.s * 27 + off;
+        rank = atomicAdd(&cnt[key], 1u);
+        kdb[key] = R.db;  // every writer of a key stores the same bin
+      }
+    }
+    __syncthreads();
+    for(int k = int(threadIdx.x); k < NK; k += WG)
+      if(cnt[k]) kbase[k] = atomicAdd(&sp.count[k / 27][kdb[k]], cnt[k]);
+    __syncthreads();
+    if(e < n) {
+      const uint32_t slot = key >= 0 ? kbase[key] + rank : atomicAdd(&sp.count[R.s][R.db], 1u);
+      const uint32_t cap = sp.cap[R.s][R.db];
+      const int64_t q = sp.start[R.s][R.db] + slot;
+      if(slot < cap) {
 #pragma unroll
         for(int d = 0; d < 3; ++d) {
-          const int NB = g.nt[d] * g.nb[d];
-          int df = global_brick(g, R.db, d) - gsrc[d];
-          df = df < 0 ? df + NB : df;
-          const int o = df == 0 ? 0 : (df == 1 ? 1 : (df == NB - 1 ? -1 : 2));
-          near = near && o != 2;
-          off = off * 3 + (o + 1);
+          sp.pos[R.s][d][q] = R.p[d];
+          sp.vel[R.s][d][q] = rv[d];
         }
-        if(near) {
-          key = R.s * 27 + off;
-          rank = atomicAdd(&cnt[key], 1u);
-          kdb[key] = R.db;  // every writer of a key stores the same bin
-        }
+        sp.id[R.s][q] = rid;
+      } else {
+        place_record(sp, m, 2, base + uint32_t(e), R, slot, counters, ovf, ovf_cap);  // overflow path
       }
-      __syncthreads();
-      for(int k = int(threadIdx.x); k < NK; k += WG)
-        if(cnt[k]) kbase[k] = atomicAdd(&sp.count[k / 27][kdb[k]], cnt[k]);
-      __syncthreads();
-      if(e < n) {
-        const uint32_t slot = key >= 0 ? kbase[key] + rank : atomicAdd(&sp.count[R.s][R.db], 1u);
-        const uint32_t cap = sp.cap[R.s][R.db];
-        const int64_t q = sp.start[R.s][R.db] + slot;
-        if(slot < cap) {
-#pragma unroll
-          for(int d = 0; d < 3; ++d) {
-            sp.pos[R.s][d][q] = R.p[d];
-            sp.vel[R.s][d][q] = rv[d];
-          }
-          sp.id[R.s][q] = rid;
-        } else {
-          place_record(sp, m, 2, base + uint32_t(e), R, slot, counters, ovf, ovf_cap);  // overflow path
-        }
-      }
-      __syncthreads();
     }
-    if(threadIdx.x == 0) m.mcount[b] = 0;
+    __syncthreads();
   }
+  if(threadIdx.x == 0) m.mcount[b] = 0;
 }
 
 __global__ void k_reset(uint32_t* counters, int which)
@@ -1886,20 +1879,12 @@ __global__ void k_reset_queues(uint32_t* counters)
   if(threadIdx.x < 8) counters[C_QUEUE + threadIdx.x] = 0;
 }
 
-// J on every lattice node += sum of the staged windows of the bricks that
-// cover it, in a fixed order.  The window of global brick gb along one axis
-// covers haloed nodes [2 + gb*br, 4 + (gb+1)*br].
-__global__ void __launch_bounds__(128)
-  k_current_gather(Geo g, const float* __restrict__ stage, int64_t stride, float* J0, float* J1, float* J2)
+// J on the nodes of lattice row (In, Jn) += sum of the staged windows of the
+// bricks that cover them, in a fixed order.  The window of global brick gb
+// along one axis covers haloed nodes [2 + gb*br, 4 + (gb+1)*br].
+__device__ inline void gather_row(const Geo& g, const float* __restrict__ stage, int64_t stride, float* J0, float* J1,
+                                  float* J2, int In, int Jn, int lane, int lanes)
 {
-  // Workgroups are dealt to the 8 XCDs round-robin by linear index; XCD x
-  // takes the x-th contiguous share of the rows instead, so the rows that
-  // share a window's cache lines (neighbouring Jn) go through one L2.
-  const int total = int(gridDim.x * gridDim.y);
-  const int lin = int(blockIdx.y * gridDim.x + blockIdx.x);
-  const int xcd = lin % 8, q8 = total / 8, r8 = total % 8;
-  const int row = xcd * q8 + min(xcd, r8) + lin / 8;
-  const int Jn = row % int(gridDim.x), In = row / int(gridDim.x);
   const int D[3] = {g.br[0] + 3, g.br[1] + 3, g.br[2] + 3};
   const int V = D[0] * D[1] * D[2];
   const int Nb[3] = {g.nt[0] * g.nb[0], g.nt[1] * g.nb[1], g.nt[2] * g.nb[2]};
@@ -1932,7 +1917,7 @@ __global__ void __launch_bounds__(128)
         const int64_t bin0 = int64_t(g.tile_lin(tx, ty, 0)) * g.bpt + (lx * g.nb[1] + ly) * g.nb[2];
         wxy[a][c] = bin0 * stride + ((a < nx ? ox[a] : 0) * D[1] + (c < ny ? oy[c] : 0)) * D[2];
       }
-    for(int K = int(threadIdx.x); K < g.L[2]; K += int(blockDim.x)) {
+    for(int K = lane; K < g.L[2]; K += lanes) {
       int64_t wz[2];
       bool vz[2];
       const int gz1 = K >= 2 ? min((K - 2) / g.br[2], Nb[2] - 1) : -1;
@@ -1981,7 +1966,7 @@ __global__ void __launch_bounds__(128)
     }
     return;
   }
-  for(int K = int(threadIdx.x); K < g.L[2]; K += int(blockDim.x)) {
+  for(int K = lane; K < g.L[2]; K += lanes) {
     float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f;
     for(int gz = min((K - 2) / g.br[2], Nb[2] - 1); K >= 2 && gz >= 0; --gz) {
       const int oz = K - (2 + gz * g.br[2]);
@@ -2006,6 +1991,44 @@ __global__ void __launch_bounds__(128)
     J1[q] = J1[q] + a1;
     J2[q] = J2[q] + a2;
   }
+}
+
+// What follows the fused step in one launch: the blocks of the mailboxes'
+// appends (which wait on memory round trips), then those of the record sets',
+// then those of the gather of the currents, none of which needs another.  All
+// three counts of blocks but the last are multiples of 8, so a block's place
+// among its kind gives its XCD: a brick's neighbours mostly run on the same one
+// (xcd_brick, as the fused step), so the appends to one destination bin's tail
+// go through one L2; XCD x gathers the x-th contiguous share of the rows, two
+// rows a block, so the rows that share a window's cache lines go through one.
+// 64^3: 20 us for the 35 us of three launches (and two gaps between them);
+// 256^3: 1.14 ms as before.  With the appends' and the gather's blocks
+// alternating on each XCD 256^3 took 1.52 ms: the gather's stream displaces the
+// partly written lines of the appends from the L2.
+constexpr int REC_BLOCKS = 128;  // they append only what spilled past full mailboxes (usually nothing)
+
+__global__ void __launch_bounds__(WG)
+  k_fused_tail(Geo g, SpParams sp, MigPtrs m, uint32_t* counters, uint32_t* ovf, int64_t ovf_cap, int span, int nappend,
+               const float* __restrict__ stage, int64_t stride, float* J0, float* J1, float* J2)
+{
+  int i = int(blockIdx.x);
+  if(i < nappend) {
+    const int b = xcd_brick(i, span);
+    if(b < g.nbricks) append_mailbox(g, sp, m, b, counters, ovf, ovf_cap);
+    return;
+  }
+  i -= nappend;
+  if(i < REC_BLOCKS) {
+    append_records(g, sp, m, i, REC_BLOCKS, counters, ovf, ovf_cap);
+    return;
+  }
+  i -= REC_BLOCKS;
+  const int rows = g.L[0] * g.L[1], total = (rows + 1) / 2;
+  const int xcd = i % 8, q8 = total / 8, r8 = total % 8;
+  const int pair = xcd * q8 + min(xcd, r8) + i / 8;
+  const int row = __builtin_amdgcn_readfirstlane(2 * pair + int(threadIdx.x) / (WG / 2));
+  if(row < rows)
+    gather_row(g, stage, stride, J0, J1, J2, row / g.L[1], row % g.L[1], int(threadIdx.x) % (WG / 2), WG / 2);
 }
 
 // in-bin counting sort by brick-local cell (layout_right), out-of-brick last
@@ -2331,26 +2354,6 @@ int launch_append(rk_world* w, int set, hipStream_t s)
   return RK_OK;
 }
 
-int launch_append_mailbox(rk_world* w, hipStream_t s)
-{
-  // one block per brick (measured faster than a capped grid)
-  const int span = xcd_span(w->g, w->g.nbricks);
-  hipLaunchKernelGGL(k_append_mailbox, dim3(xcd_grid(w->g.nbricks, span)), dim3(WG), 0, s, w->g, make_sp(w),
-                     make_mig(w), w->g.nbricks, w->counters, w->ovf_list, w->ovf_cap, span);
-  RK_HIP(hipGetLastError());
-  return RK_OK;
-}
-
-int launch_append_records(rk_world* w, hipStream_t s)
-{
-  // the sets hold only what spilled past full mailboxes (usually nothing):
-  // a small grid, since every workgroup signs off with a fence and an atomic
-  hipLaunchKernelGGL(k_append_records, dim3(64, 2), dim3(WG), 0, s, w->g, make_sp(w), make_mig(w), w->counters,
-                     w->ovf_list, w->ovf_cap);
-  RK_HIP(hipGetLastError());
-  return RK_OK;
-}
-
 int launch_reset_counter(rk_world* w, int which, hipStream_t s)
 {
   hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, s, w->counters, which);
@@ -2435,10 +2438,14 @@ int launch_fused(rk_world* w, hipStream_t s, const WallSet* walls, const rk_refl
   return RK_OK;
 }
 
-int launch_current_gather(rk_world* w, hipStream_t s)
+int launch_fused_tail(rk_world* w, hipStream_t s)
 {
-  hipLaunchKernelGGL(k_current_gather, dim3(unsigned(w->g.L[1]), unsigned(w->g.L[0])), dim3(128), 0, s, w->g,
-                     w->jstage, w->jstage_stride, w->J[0], w->J[1], w->J[2]);
+  const Geo& g = w->g;
+  const int span = xcd_span(g, g.nbricks);
+  const int nappend = int(xcd_grid(g.nbricks, span));  // a multiple of 8
+  const int pairs = (g.L[0] * g.L[1] + 1) / 2;
+  hipLaunchKernelGGL(k_fused_tail, dim3(unsigned(nappend + REC_BLOCKS + pairs)), dim3(WG), 0, s, g, make_sp(w), make_mig(w), w->counters,
+                     w->ovf_list, w->ovf_cap, span, nappend, w->jstage, w->jstage_stride, w->J[0], w->J[1], w->J[2]);
   RK_HIP(hipGetLastError());
   return RK_OK;
 }

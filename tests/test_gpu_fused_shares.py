@@ -3,7 +3,8 @@ contiguous share of 64-particle chunks and compacts it in place.  Bricks hold
 the particle counts where that can go wrong (none, one, around one chunk,
 around one chunk per wave, a remainder past it), three species (odd ones deal
 their shares in reverse), and one brick whose particles all leave (more of
-them than its 64-record mailbox holds).  One lap against the oracle with the
+them than its 64-record mailbox holds).  The last shape has an odd number of
+lattice rows (the gather that follows takes them in pairs).  One lap against the oracle with the
 bars of the other one-lap tests: particles bit-exact, fields within 1e-6."""
 
 import numpy as np
@@ -42,7 +43,8 @@ def share_inputs(nt, n, brick, seed):
     return tiles
 
 
-@pytest.mark.parametrize("n,brick", [((8, 8, 16), (8, 8, 8)), ((4, 4, 8), (4, 4, 4)), ((6, 7, 10), (6, 7, 5))])
+@pytest.mark.parametrize("n,brick", [((8, 8, 16), (8, 8, 8)), ((4, 4, 8), (4, 4, 4)), ((6, 7, 10), (6, 7, 5)),
+                                     ((5, 7, 10), (5, 7, 5))])
 @pytest.mark.parametrize("pusher", ["boris", "higuera_cary", "faraday"])
 def test_one_lap_parity_share_edges(orc, n, brick, pusher):
     nt = (3, 3, 1)
