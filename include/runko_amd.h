@@ -239,6 +239,14 @@ int rk_read_walls(rk_world* w, rk_reflector_wall* out, int32_t n_walls, void* st
  * node as rk_push_e then rk_add_current).  Batched form of that pair. */
 int rk_push_e_add_current(rk_world* w, int32_t tile, void* stream);
 
+/* Batched pairs of an update of every tile and the exchange after it, fewer
+ * launches: push_half_b then comm emf_B, rk_push_e_add_current then comm emf_E,
+ * comm emf_J_exchange then comm emf_J.  The fields hold the same values as
+ * after the two calls. */
+int rk_push_half_b_comm(rk_world* w, void* stream);
+int rk_push_e_add_current_comm(rk_world* w, void* stream);
+int rk_exchange_current(rk_world* w, void* stream);
+
 /* Kernel timing: when enabled, every launch is bracketed by HIP events on its
  * stream, accumulated per category; rk_profile_read (synchronous) returns and
  * clears the totals.  Categories: 0 fused particle step kernel, 1 push,

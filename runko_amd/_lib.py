@@ -117,6 +117,8 @@ def lib():
     L.rk_advance_walls.argtypes = [vp, vp]
     L.rk_read_walls.argtypes = [vp, vp, i32, vp]
     L.rk_push_e_add_current.argtypes = [vp, i32, vp]
+    for name in ["rk_push_half_b_comm", "rk_push_e_add_current_comm", "rk_exchange_current"]:
+        getattr(L, name).argtypes = [vp, vp]
     L.rk_profile_enable.argtypes = [vp, i32]
     L.rk_profile_read.argtypes = [vp, vp, vp]
     L.rk_comm_local.argtypes = [vp, i32, vp]
@@ -171,7 +173,7 @@ EXPORTED = [
     "rk_profile_read", "rk_world_set_mailbox", "rk_world_set_current_staging", "rk_reflect_particles",
     "rk_apply_edge_bc", "rk_diff_create", "rk_diff_create_ensemble", "rk_diff_destroy", "rk_diff_step", "rk_diff_step_adjoint",
     "rk_diff_error_count", "rk_snapshot_fields", "rk_snapshot_spectra", "rk_interpolate_at",
-    "rk_world_set_schemes",
+    "rk_world_set_schemes", "rk_push_half_b_comm", "rk_push_e_add_current_comm", "rk_exchange_current",
 ]
 
 PROF_CATEGORIES = ["fused_particle_step", "push", "deposit", "pack", "append", "fdtd", "filter", "ghost", "other"]

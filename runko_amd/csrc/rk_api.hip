@@ -427,7 +427,20 @@ int rk_push_half_b(rk_world* w, int32_t tile, void* stream)
   ProfScope ps(w, 5, S(stream));
   const float dt = static_cast<float>(w->d.cfl / 2);
   if(w->stencil_on) return launch_curl_b_stencil(w, r0, r1, dt, S(stream));
-  return launch_curl_b(w, r0, r1, dt, S(stream));
+  return launch_curl_b(w, r0, r1, dt, false, S(stream));
+}
+
+int rk_push_half_b_comm(rk_world* w, void* stream)
+{
+  if(w && (w->stencil_on || !w->g.periodic)) {
+    if(int rc = rk_push_half_b(w, -1, stream)) return rc;
+    return rk_comm_local(w, RK_COMM_EMF_B, stream);
+  }
+  if(int rc = check_tile(w, -1)) return rc;
+  int r0[3], r1[3];
+  interior(w, -1, r0, r1);
+  ProfScope ps(w, 5, S(stream));
+  return launch_curl_b(w, r0, r1, static_cast<float>(w->d.cfl / 2), true, S(stream));
 }
 
 int rk_world_set_schemes(rk_world* w, int32_t particle_pusher, const float* stencil)
@@ -446,7 +459,7 @@ int rk_push_e(rk_world* w, int32_t tile, void* stream)
   int r0[3], r1[3];
   interior(w, tile, r0, r1);
   ProfScope ps(w, 5, S(stream));
-  return launch_curl_e(w, r0, r1, static_cast<float>(w->d.cfl), false, S(stream));
+  return launch_curl_e(w, r0, r1, static_cast<float>(w->d.cfl), false, false, S(stream));
 }
 
 int rk_push_e_add_current(rk_world* w, int32_t tile, void* stream)
@@ -456,7 +469,30 @@ int rk_push_e_add_current(rk_world* w, int32_t tile, void* stream)
   int r0[3], r1[3];
   interior(w, tile, r0, r1);
   ProfScope ps(w, 5, S(stream));
-  return launch_curl_e(w, r0, r1, static_cast<float>(w->d.cfl), true, S(stream));
+  return launch_curl_e(w, r0, r1, static_cast<float>(w->d.cfl), true, false, S(stream));
+}
+
+int rk_push_e_add_current_comm(rk_world* w, void* stream)
+{
+  if(w && !w->g.periodic) {
+    if(int rc = rk_push_e_add_current(w, -1, stream)) return rc;
+    return rk_comm_local(w, RK_COMM_EMF_E, stream);
+  }
+  if(int rc = check_tile(w, -1)) return rc;
+  close_j(w);
+  int r0[3], r1[3];
+  interior(w, -1, r0, r1);
+  ProfScope ps(w, 5, S(stream));
+  return launch_curl_e(w, r0, r1, static_cast<float>(w->d.cfl), true, true, S(stream));
+}
+
+int rk_exchange_current(rk_world* w, void* stream)
+{
+  if(int rc = check_tile(w, -1)) return rc;
+  if(!w->g.periodic) return fail(RK_EINVAL, "exchange_current needs a tile grid (stand-alone tile)");
+  close_j(w);
+  ProfScope ps(w, 7, S(stream));
+  return launch_ghost_fold(w, w->J, true, S(stream));
 }
 
 int rk_add_current(rk_world* w, int32_t tile, void* stream)
@@ -677,7 +713,7 @@ int rk_comm_local(rk_world* w, int32_t mode, void* stream)
     case RK_COMM_EMF_E: return launch_ghost_copy(w, w->E, s);
     case RK_COMM_EMF_B: return launch_ghost_copy(w, w->B, s);
     case RK_COMM_EMF_J: close_j(w); return launch_ghost_copy(w, w->J, s);
-    case RK_COMM_EMF_J_EXCHANGE: close_j(w); return launch_ghost_fold(w, w->J, s);
+    case RK_COMM_EMF_J_EXCHANGE: close_j(w); return launch_ghost_fold(w, w->J, false, s);
     case RK_COMM_PIC_PARTICLE: {
       if(int rc = check_particles(w)) return rc;
       if(int rc = launch_append(w, 0, s)) return rc;

@@ -36,8 +36,36 @@ inline dim3 region_grid(const Region& r)
   return dim3((ez + BX - 1) / BX, (ey + BY - 1) / BY, ex);
 }
 
+// A periodic world with at least 2 * HALO cells along every axis: an interior
+// node has at most one image in the ghost shell along an axis, ghost_step away.
+// A kernel that computes whole fields stores a node's new value into its (up to
+// 7) images as well (`ghosts`), so no launch has to copy the ghost shell after
+// it: at 64^3 such a copy takes 5 us, as long as the kernel before it.
+bool ghosts_in_pass(const Geo& g)
+{
+  return g.periodic && g.N[0] >= 2 * HALO && g.N[1] >= 2 * HALO && g.N[2] >= 2 * HALO;
+}
+
+__device__ inline int ghost_step(int c, int N) { return c < 2 * HALO ? N : (c >= N ? -N : 0); }
+
+__device__ inline void put_ghosts(const Geo& g, int i, int j, int k, uint32_t c, float* F0, float* F1, float* F2,
+                                  float v0, float v1, float v2)
+{
+  const int d0 = ghost_step(i, g.N[0]) * g.L[1] * g.L[2], d1 = ghost_step(j, g.N[1]) * g.L[2];
+  const int d2 = ghost_step(k, g.N[2]);
+  if((d0 | d1 | d2) == 0) return;
+#pragma unroll 1
+  for(int n = 1; n < 8; ++n) {
+    if(((n & 4) && !d0) || ((n & 2) && !d1) || ((n & 1) && !d2)) continue;
+    const uint32_t q = c + uint32_t((n & 4 ? d0 : 0) + (n & 2 ? d1 : 0) + (n & 1 ? d2 : 0));
+    F0[q] = v0;
+    F1[q] = v1;
+    F2[q] = v2;
+  }
+}
+
 __global__ void __launch_bounds__(BX* BY)
-  k_curl_b(Geo g, Region r, float dt, const float* __restrict__ Ex, const float* __restrict__ Ey,
+  k_curl_b(Geo g, Region r, float dt, int ghosts, const float* __restrict__ Ex, const float* __restrict__ Ey,
            const float* __restrict__ Ez, float* __restrict__ Bx, float* __restrict__ By,
            float* __restrict__ Bz)
 {
@@ -50,13 +78,17 @@ __global__ void __launch_bounds__(BX* BY)
   const float ex = Ex[c], ey = Ey[c], ez = Ez[c];
   const float DkEy = Ey[c + 1] - ey;
   const float DjEz = Ez[c + sj] - ez;
-  Bx[c] = Bx[c] + dt * (DkEy - DjEz);
+  const float bx = Bx[c] + dt * (DkEy - DjEz);
   const float DiEz = Ez[c + si] - ez;
   const float DkEx = Ex[c + 1] - ex;
-  By[c] = By[c] + dt * (DiEz - DkEx);
+  const float by = By[c] + dt * (DiEz - DkEx);
   const float DjEx = Ex[c + sj] - ex;
   const float DiEy = Ey[c + si] - ey;
-  Bz[c] = Bz[c] + dt * (DjEx - DiEy);
+  const float bz = Bz[c] + dt * (DjEx - DiEy);
+  Bx[c] = bx;
+  By[c] = by;
+  Bz[c] = bz;
+  if(ghosts) put_ghosts(g, i, j, k, c, Bx, By, Bz, bx, by, bz);
 }
 
 // push_b_stencil, src/runko/emf/yee_lattice_stencil.c++:17-297: each
@@ -205,7 +237,7 @@ __global__ void __launch_bounds__(BX* BY)
 
 template<bool ADDJ>
 __global__ void __launch_bounds__(BX* BY)
-  k_curl_e(Geo g, Region r, float dt, const float* __restrict__ Bx, const float* __restrict__ By,
+  k_curl_e(Geo g, Region r, float dt, int ghosts, const float* __restrict__ Bx, const float* __restrict__ By,
            const float* __restrict__ Bz, float* __restrict__ Ex, float* __restrict__ Ey,
            float* __restrict__ Ez, const float* __restrict__ Jx, const float* __restrict__ Jy,
            const float* __restrict__ Jz)
@@ -234,6 +266,7 @@ __global__ void __launch_bounds__(BX* BY)
   Ex[c] = ex;
   Ey[c] = ey;
   Ez[c] = ez;
+  if(ghosts) put_ghosts(g, i, j, k, c, Ex, Ey, Ez, ex, ey, ez);
 }
 
 __global__ void __launch_bounds__(BX* BY)
@@ -575,6 +608,72 @@ __global__ void __launch_bounds__(64) k_ghost_copy(Geo g, int nrows, float* F0, 
   }
 }
 
+// periodic ghost fold (J_exchange): interior node += all of its ghost images,
+// in the order of the offsets (x slowest); with `copy` its images then take the
+// sum (the ghost copy that follows the fold: the nodes that have images are the
+// same).  A world with images on one axis side at most (ghosts_in_pass); only
+// the nodes within HALO layers of a face are touched, a component per
+// blockIdx.y: the first nrows workgroups take the whole z rows whose i or j lies
+// in those layers (all j of the layers of i, then the layers of j of the other
+// i), the workgroups after them the z layers of the other rows, six lanes a row.
+// Small worlds are bound by latency, also that of fetching the code: 64^3 took
+// 17 us with all components, the general case below and a workgroup per row in
+// one kernel, and the copy 5 us; @@FOLD@@
+__global__ void __launch_bounds__(256) k_fold_copy(Geo g, int nrows, int copy, float* F0, float* F1, float* F2)
+{
+  float* const F = blockIdx.y == 0 ? F0 : (blockIdx.y == 1 ? F1 : F2);
+  const int blk = int(blockIdx.x), tid = int(threadIdx.x);
+  auto layer = [](int t, int N) { return t < HALO ? HALO + t : N + t - HALO; };  // t-th layer node of an axis
+  int i, j, k0 = HALO + tid, k1 = HALO + g.N[2];
+  if(blk < nrows) {
+    const int nA = 2 * HALO * g.N[1];
+    if(blk < nA) {
+      const int t = blk / g.N[1];
+      i = layer(t, g.N[0]);
+      j = HALO + blk - t * g.N[1];
+    } else {
+      const int t = (blk - nA) / (2 * HALO);
+      i = 2 * HALO + t;
+      j = layer(blk - nA - t * 2 * HALO, g.N[1]);
+    }
+  } else {
+    const int per = int(blockDim.x) / (2 * HALO), r = tid / (2 * HALO);
+    const uint32_t other = uint32_t(g.N[1] - 2 * HALO), row = uint32_t(blk - nrows) * uint32_t(per) + uint32_t(r);
+    if(r >= per || row >= uint32_t(g.N[0] - 2 * HALO) * other) return;
+    i = 2 * HALO + int(row / other);
+    j = 2 * HALO + int(row % other);
+    k0 = layer(tid - r * 2 * HALO, g.N[2]);
+    k1 = k0 + 1;
+  }
+  const int d0 = ghost_step(i, g.N[0]) * g.L[1] * g.L[2], d1 = ghost_step(j, g.N[1]) * g.L[2];
+  for(int k = k0; k < k1; k += int(blockDim.x)) {
+    const int d2 = ghost_step(k, g.N[2]);
+    if((d0 | d1 | d2) == 0) continue;
+    const uint32_t c = g.at(i, j, k);
+    uint32_t q[8];
+    float v[8];
+#pragma unroll
+    for(int n = 0; n < 8; ++n) {
+      q[n] = c + uint32_t((n & 4 ? d0 : 0) + (n & 2 ? d1 : 0) + (n & 1 ? d2 : 0));
+      v[n] = F[q[n]];  // an image that is not there reads another of the eight
+    }
+    auto there = [&](int n) { return (!(n & 4) || d0 != 0) && (!(n & 2) || d1 != 0) && (!(n & 1) || d2 != 0); };
+    float sum = v[0];
+#pragma unroll
+    for(int n = 1; n < 8; ++n) {
+      asm volatile("" : "+v"(v[n]));  // keeps the loads together, ahead of the conditions
+      const float t = sum + v[n];
+      sum = there(n) ? t : sum;
+    }
+    F[c] = sum;
+    if(copy) {
+#pragma unroll
+      for(int n = 1; n < 8; ++n)
+        if(there(n)) F[q[n]] = sum;
+    }
+  }
+}
+
 // images of an interior coordinate c in the ghost shell: c-N (c >= N) and c+N (c < 2*HALO)
 __device__ inline int images(int c, int N, int out[3])
 {
@@ -585,52 +684,19 @@ __device__ inline int images(int c, int N, int out[3])
   return m;
 }
 
-// periodic ghost fold (J_exchange): interior node += all of its ghost images
-__global__ void __launch_bounds__(256) k_ghost_fold(Geo g, float* F0, float* F1, float* F2)
+// the fold on a world with fewer than 2 * HALO cells along an axis, where a
+// node may have two images along it; a workgroup per row
+__global__ void __launch_bounds__(64) k_fold_thin(Geo g, float* F0, float* F1, float* F2)
 {
-  const int j = HALO + int(blockIdx.x);
-  const int i = HALO + int(blockIdx.y);
+  const int j = HALO + int(blockIdx.x), i = HALO + int(blockIdx.y);
   int ii[3], jj[3], kk[3];
   const int mi = images(i, g.N[0], ii);
   const int mj = images(j, g.N[1], jj);
-  // with N >= 2*HALO per axis a node has at most two images per axis: all of
-  // its (up to 7) ghost images are addressed first and loaded together, then
-  // added in the order of the general loop below (bit-identical)
-  const bool two = g.N[0] >= 2 * HALO && g.N[1] >= 2 * HALO && g.N[2] >= 2 * HALO;
-  auto fold = [&](int k) {
+  for(int k = HALO + int(threadIdx.x); k < g.N[2] + HALO; k += int(blockDim.x)) {
     const int mk = images(k, g.N[2], kk);
-    if(mi * mj * mk == 1) return;
+    if(mi * mj * mk == 1) continue;
     const uint32_t c = g.at(i, j, k);
     float s0 = F0[c], s1 = F1[c], s2 = F2[c];
-    if(two) {
-      float v[8][3];
-#pragma unroll
-      for(int a = 0; a < 2; ++a)
-#pragma unroll
-        for(int b = 0; b < 2; ++b)
-#pragma unroll
-          for(int e = 0; e < 2; ++e) {
-            const bool ok = a < mi && b < mj && e < mk && (a | b | e) != 0;
-            const uint32_t q = ok ? g.at(ii[a], jj[b], kk[e]) : c;
-            const int n = (a * 2 + b) * 2 + e;
-            v[n][0] = F0[q];
-            v[n][1] = F1[q];
-            v[n][2] = F2[q];
-          }
-#pragma unroll
-      for(int n = 1; n < 8; ++n) {
-        const int a = n >> 2, b = (n >> 1) & 1, e = n & 1;
-        const bool ok = a < mi && b < mj && e < mk;
-        const float t0 = s0 + v[n][0], t1 = s1 + v[n][1], t2 = s2 + v[n][2];
-        s0 = ok ? t0 : s0;
-        s1 = ok ? t1 : s1;
-        s2 = ok ? t2 : s2;
-      }
-      F0[c] = s0;
-      F1[c] = s1;
-      F2[c] = s2;
-      return;
-    }
     for(int a = 0; a < mi; ++a)
       for(int b = 0; b < mj; ++b)
         for(int e = 0; e < mk; ++e) {
@@ -643,15 +709,6 @@ __global__ void __launch_bounds__(256) k_ghost_fold(Geo g, float* F0, float* F1,
     F0[c] = s0;
     F1[c] = s1;
     F2[c] = s2;
-  };
-  if(mi * mj > 1) {
-    for(int k = HALO + int(threadIdx.x); k < g.N[2] + HALO; k += int(blockDim.x)) fold(k);
-  } else {
-    const int t = int(threadIdx.x);
-    if(t < 2 * HALO) {
-      const int k = t < HALO ? HALO + t : g.N[2] + t - HALO;
-      if(k >= HALO && k < g.N[2] + HALO && (t < HALO || k >= HALO + HALO)) fold(k);
-    }
   }
 }
 
@@ -711,14 +768,16 @@ bool empty(const Region& r) { return r.r1[0] <= r.r0[0] || r.r1[1] <= r.r0[1] ||
 
 }  // namespace
 
-int launch_curl_b(rk_world* w, const int r0[3], const int r1[3], float dt, hipStream_t s)
+// ghosts: the ghost shell holds the images of the new interior afterwards
+int launch_curl_b(rk_world* w, const int r0[3], const int r1[3], float dt, bool ghosts, hipStream_t s)
 {
   const Region r = make_region(r0, r1);
   if(empty(r)) return RK_OK;
-  hipLaunchKernelGGL(k_curl_b, region_grid(r), dim3(BX, BY), 0, s, w->g, r, dt, w->E[0], w->E[1], w->E[2],
+  const bool in_pass = ghosts && ghosts_in_pass(w->g);
+  hipLaunchKernelGGL(k_curl_b, region_grid(r), dim3(BX, BY), 0, s, w->g, r, dt, int(in_pass), w->E[0], w->E[1], w->E[2],
                      w->B[0], w->B[1], w->B[2]);
   RK_HIP(hipGetLastError());
-  return RK_OK;
+  return ghosts && !in_pass ? launch_ghost_copy(w, w->B, s) : RK_OK;
 }
 
 int launch_curl_b_stencil(rk_world* w, const int r0[3], const int r1[3], float dt, hipStream_t s)
@@ -735,18 +794,15 @@ int launch_curl_b_stencil(rk_world* w, const int r0[3], const int r1[3], float d
   return RK_OK;
 }
 
-int launch_curl_e(rk_world* w, const int r0[3], const int r1[3], float dt, bool add_j, hipStream_t s)
+int launch_curl_e(rk_world* w, const int r0[3], const int r1[3], float dt, bool add_j, bool ghosts, hipStream_t s)
 {
   const Region r = make_region(r0, r1);
   if(empty(r)) return RK_OK;
-  if(add_j)
-    hipLaunchKernelGGL(k_curl_e<true>, region_grid(r), dim3(BX, BY), 0, s, w->g, r, dt, w->B[0], w->B[1],
-                       w->B[2], w->E[0], w->E[1], w->E[2], w->J[0], w->J[1], w->J[2]);
-  else
-    hipLaunchKernelGGL(k_curl_e<false>, region_grid(r), dim3(BX, BY), 0, s, w->g, r, dt, w->B[0], w->B[1],
-                       w->B[2], w->E[0], w->E[1], w->E[2], w->J[0], w->J[1], w->J[2]);
+  const bool in_pass = ghosts && ghosts_in_pass(w->g);
+  hipLaunchKernelGGL(add_j ? k_curl_e<true> : k_curl_e<false>, region_grid(r), dim3(BX, BY), 0, s, w->g, r, dt,
+                     int(in_pass), w->B[0], w->B[1], w->B[2], w->E[0], w->E[1], w->E[2], w->J[0], w->J[1], w->J[2]);
   RK_HIP(hipGetLastError());
-  return RK_OK;
+  return ghosts && !in_pass ? launch_ghost_copy(w, w->E, s) : RK_OK;
 }
 
 int launch_add_current(rk_world* w, const int r0[3], const int r1[3], hipStream_t s)
@@ -803,9 +859,21 @@ int launch_ghost_copy(rk_world* w, float* const F[3], hipStream_t s)
   return RK_OK;
 }
 
-int launch_ghost_fold(rk_world* w, float* const F[3], hipStream_t s)
+// copy: the ghost copy after the fold too
+int launch_ghost_fold(rk_world* w, float* const F[3], bool copy, hipStream_t s)
 {
-  hipLaunchKernelGGL(k_ghost_fold, dim3(w->g.N[1], w->g.N[0]), dim3(64), 0, s, w->g, F[0], F[1], F[2]);
+  const Geo& g = w->g;
+  if(!ghosts_in_pass(g)) {
+    hipLaunchKernelGGL(k_fold_thin, dim3(g.N[1], g.N[0]), dim3(64), 0, s, g, F[0], F[1], F[2]);
+    RK_HIP(hipGetLastError());
+    return copy ? launch_ghost_copy(w, F, s) : RK_OK;
+  }
+  const int threads = 64 * std::min(4, (g.N[2] + 63) / 64);
+  const int nrows = 2 * HALO * (g.N[1] + g.N[0] - 2 * HALO);
+  const int64_t others = int64_t(g.N[0] - 2 * HALO) * (g.N[1] - 2 * HALO);
+  const int per = threads / (2 * HALO);
+  hipLaunchKernelGGL(k_fold_copy, dim3(unsigned(nrows + (others + per - 1) / per), 3), dim3(unsigned(threads)), 0, s, g,
+                     nrows, int(copy), F[0], F[1], F[2]);
   RK_HIP(hipGetLastError());
   return RK_OK;
 }

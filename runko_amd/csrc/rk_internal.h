@@ -230,13 +230,13 @@ int hip_fail(hipError_t e, const char* where);
   } while(0)
 
 // launchers implemented in rk_fields.hip / rk_particles.hip
-int launch_curl_b(rk_world* w, const int r0[3], const int r1[3], float dt, hipStream_t s);
+int launch_curl_b(rk_world* w, const int r0[3], const int r1[3], float dt, bool ghosts, hipStream_t s);
 int launch_curl_b_stencil(rk_world* w, const int r0[3], const int r1[3], float dt, hipStream_t s);
-int launch_curl_e(rk_world* w, const int r0[3], const int r1[3], float dt, bool add_j, hipStream_t s);
+int launch_curl_e(rk_world* w, const int r0[3], const int r1[3], float dt, bool add_j, bool ghosts, hipStream_t s);
 int launch_add_current(rk_world* w, const int r0[3], const int r1[3], hipStream_t s);
 int launch_filter(rk_world* w, const int r0[3], const int r1[3], hipStream_t s);
 int launch_ghost_copy(rk_world* w, float* const F[3], hipStream_t s);
-int launch_ghost_fold(rk_world* w, float* const F[3], hipStream_t s);
+int launch_ghost_fold(rk_world* w, float* const F[3], bool copy, hipStream_t s);
 int launch_fill(float* const F[3], int64_t n, float v, hipStream_t s);
 int field_energies(rk_world* w, const int r0[3], const int r1[3], double out[2], hipStream_t s);
 

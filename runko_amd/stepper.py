@@ -33,17 +33,13 @@ class BatchedLap:
 
     def __call__(self):
         w = self.w
-        w.call("rk_push_half_b", -1)
-        w.comm_local(int(comm_mode.emf_B))
+        w.push_half_b_comm()
         w.particle_step_fused()
-        w.comm_local(int(comm_mode.emf_J_exchange))
-        w.comm_local(int(comm_mode.emf_J))
+        w.exchange_current()
         # filter, comm J, filter, filter (pic.py:208-212) as one call
         w.filter_current_passes(self.filter_passes)
-        w.call("rk_push_half_b", -1)
-        w.comm_local(int(comm_mode.emf_B))
-        w.call("rk_push_e_add_current", -1)
-        w.comm_local(int(comm_mode.emf_E))
+        w.push_half_b_comm()
+        w.push_e_add_current_comm()
 
     def settle(self):
         """Synchronous check after a lap: bins that overflowed are repacked and
@@ -224,8 +220,11 @@ class ShockLap:
             self._each("rk_pack_outgoing_particles")
             w.comm_local(int(comm_mode.pic_particle))
             self._each("rk_deposit_current")
-        w.comm_local(int(comm_mode.emf_J_exchange))
-        w.comm_local(int(comm_mode.emf_J))
+        if self.tiles is None:
+            w.exchange_current()
+        else:
+            w.comm_local(int(comm_mode.emf_J_exchange))
+            w.comm_local(int(comm_mode.emf_J))
         self._bcs(comm_mode.emf_J)
         if self.tiles is None and self.filter_passes == 3 and w.periodic and w.current_filter == "binomial2":
             # three passes with no ghost sync between them: one launch reading

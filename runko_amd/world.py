@@ -337,6 +337,18 @@ class World:
         launch for three binomial2 passes on a periodic world)."""
         L.check(L.lib().rk_filter_current_passes(self.h, int(passes), _stream()))
 
+    def push_half_b_comm(self):
+        """push_half_b on every tile, then comm_local(emf_B), in one launch."""
+        L.check(L.lib().rk_push_half_b_comm(self.h, _stream()))
+
+    def push_e_add_current_comm(self):
+        """push_e and add_current on every tile, then comm_local(emf_E), in one launch."""
+        L.check(L.lib().rk_push_e_add_current_comm(self.h, _stream()))
+
+    def exchange_current(self):
+        """comm_local(emf_J_exchange), then comm_local(emf_J), in one launch."""
+        L.check(L.lib().rk_exchange_current(self.h, _stream()))
+
     def comm_local(self, mode):
         rc = L.lib().rk_comm_local(self.h, int(mode), _stream())
         if rc == L.RK_EOVERFLOW:
