@@ -17,6 +17,7 @@
 
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 
 namespace rk {
 
@@ -104,7 +105,9 @@ struct StencilM {
 // sum over n, col of M[n][col] * diff(n, col) in the reference's order;
 // at(ax, o1, o2) reads the field at offset ax along the derivative's axis a
 // and o1, o2 along the cyclic perpendicular axes (a+1)%3, (a+2)%3
-template<class At>
+// AXIAL: rows 1 and 2 have coefficients on the axial line only; their other
+// terms, 0 times a finite difference each, are left out
+template<bool AXIAL, class At>
 __device__ inline float stencil_sum(At&& at, const float (&M)[3][5])
 {
   float sum = 0.0f;
@@ -112,7 +115,7 @@ __device__ inline float stencil_sum(At&& at, const float (&M)[3][5])
   for(int n = 0; n < 3; ++n) {
     const int hi = n + 1, lo = -n;
 #pragma unroll
-    for(int col = 0; col < 5; ++col) {
+    for(int col = 0; col < (AXIAL && n > 0 ? 1 : 5); ++col) {
       float diff;
       if(col == 0) {
         diff = at(hi, 0, 0) - at(lo, 0, 0);
@@ -132,11 +135,11 @@ __device__ inline float stencil_sum(At&& at, const float (&M)[3][5])
 
 // The stencil reads offsets -2..3 along the derivative's axis and -2..2
 // across it (324 reads of E per cell).  A block (BX cells along z, BY along
-// y) marches through SCH x planes, keeping the last six planes of E over
+// y) marches through xseg x planes, keeping the last six planes of E over
 // y, z in [start-2, end+3) in an LDS ring: each plane is read from memory
 // once per block, in rows along z, and every cell takes its six derivatives
 // from the ring.
-constexpr int SSY = BY + 5, SSZ = BX + 5, SPL = SSY * SSZ, SCH = 32;
+constexpr int SSY = BY + 5, SSZ = BX + 5, SPL = SSY * SSZ;
 
 // One plane of the ring is 3 * SSY rows of SSZ floats; wave w of the block
 // moves rows w, w + 4, ... (lanes along z), through registers so the loads
@@ -164,8 +167,10 @@ __device__ inline void stencil_load(const Geo& g, float (&v)[SROWS][SLANES], int
   }
 }
 
-__device__ inline void stencil_store(float (&E)[3][6 * SPL], int slot, const float (&v)[SROWS][SLANES])
+// true if a value of this lane is an infinity or a NaN
+__device__ inline bool stencil_store(float (&E)[3][6 * SPL], int slot, const float (&v)[SROWS][SLANES])
 {
+  float zero = 0.0f;
   const int wave = __builtin_amdgcn_readfirstlane((int(threadIdx.y) * BX + int(threadIdx.x)) / 64);
   const int lane = int(threadIdx.x) % 64;
 #pragma unroll
@@ -174,15 +179,18 @@ __device__ inline void stencil_store(float (&E)[3][6 * SPL], int slot, const flo
 #pragma unroll
     for(int h = 0; h < SLANES; ++h)
       if(row < 3 * SSY && lane + 64 * h < SSZ) E[c][slot * SPL + y * SSZ + lane + 64 * h] = v[q][h];
+#pragma unroll
+    for(int h = 0; h < SLANES; ++h) zero = zero + v[q][h] * 0.0f;
   }
+  return !(zero == 0.0f);
 }
 
 // derivative along axis A of the staged component Ec at the ring cell `cell`;
 // sb[d] is the ring offset of plane x + d - 2
-template<int A>
+template<int A, bool AXIAL>
 __device__ inline float stencil_lds(const float* Ec, const int (&sb)[6], int cell, const float (&M)[3][5])
 {
-  return stencil_sum(
+  return stencil_sum<AXIAL>(
     [&](int ax, int o1, int o2) {
       int d[3];
       d[A] = ax;
@@ -193,42 +201,56 @@ __device__ inline float stencil_lds(const float* Ec, const int (&sb)[6], int cel
     M);
 }
 
+// What bounds it: LDS reads, 324 per cell, and, on a world whose whole
+// segments are too few blocks, latency.  `axial` (the coefficients of the
+// reference's shock configuration, projects/pic-shock/3d_shock.ini:48-70, are of
+// that form) takes 132 reads as long as every value that the block has staged
+// is finite.  512 x 64 x 64 cells: 130 us in segments of 32 planes (256 blocks),
+// 89 us in segments of 8, 63 us axial.
 __global__ void __launch_bounds__(BX* BY)
-  k_curl_b_stencil(Geo g, Region r, float dt, StencilM S, const float* __restrict__ Ex,
+  k_curl_b_stencil(Geo g, Region r, float dt, StencilM S, int xseg, int axial, const float* __restrict__ Ex,
                    const float* __restrict__ Ey, const float* __restrict__ Ez, float* __restrict__ Bx,
                    float* __restrict__ By, float* __restrict__ Bz)
 {
   __shared__ float E[3][6 * SPL];
+  __shared__ int full;  // take all terms
   const int k0 = r.r0[2] + int(blockIdx.x) * BX, j0 = r.r0[1] + int(blockIdx.y) * BY;
-  const int i0 = r.r0[0] + int(blockIdx.z) * SCH, i1 = min(r.r1[0], i0 + SCH);
+  const int i0 = r.r0[0] + int(blockIdx.z) * xseg, i1 = min(r.r1[0], i0 + xseg);
   const int k = k0 + int(threadIdx.x), j = j0 + int(threadIdx.y);
   const bool active = k < r.r1[2] && j < r.r1[1];
   const int cell = (2 + int(threadIdx.y)) * SSZ + 2 + int(threadIdx.x);
   float v[SROWS][SLANES];
+  if(threadIdx.x == 0 && threadIdx.y == 0) full = !axial;
+  __syncthreads();
   for(int p = 0; p < 5; ++p) {
     stencil_load(g, v, i0 - 2 + p, j0, k0, Ex, Ey, Ez);
-    stencil_store(E, p, v);
+    if(stencil_store(E, p, v)) full = 1;
   }
   stencil_load(g, v, i0 + 3, j0, k0, Ex, Ey, Ez);
   int base = 0;  // ring slot of plane i - 2
   for(int i = i0; i < i1; ++i) {
-    stencil_store(E, base == 0 ? 5 : base - 1, v);
+    if(stencil_store(E, base == 0 ? 5 : base - 1, v)) full = 1;
     __syncthreads();
     if(i + 1 < i1) stencil_load(g, v, i + 4, j0, k0, Ex, Ey, Ez);
-    if(active) {
-      int sb[6];
+    int sb[6];
 #pragma unroll
-      for(int d = 0; d < 6; ++d) sb[d] = (base + d < 6 ? base + d : base + d - 6) * SPL;
-      const int64_t c = g.at(i, j, k);
-      const float DzEy = stencil_lds<2>(E[1], sb, cell, S.M[2]);
-      const float DyEz = stencil_lds<1>(E[2], sb, cell, S.M[1]);
+    for(int d = 0; d < 6; ++d) sb[d] = (base + d < 6 ? base + d : base + d - 6) * SPL;
+    const uint32_t c = g.at(i, j, k);
+    auto update = [&](auto ax) {
+      constexpr bool AX = decltype(ax)::value;
+      const float DzEy = stencil_lds<2, AX>(E[1], sb, cell, S.M[2]);
+      const float DyEz = stencil_lds<1, AX>(E[2], sb, cell, S.M[1]);
       Bx[c] = Bx[c] + dt * (DzEy - DyEz);
-      const float DxEz = stencil_lds<0>(E[2], sb, cell, S.M[0]);
-      const float DzEx = stencil_lds<2>(E[0], sb, cell, S.M[2]);
+      const float DxEz = stencil_lds<0, AX>(E[2], sb, cell, S.M[0]);
+      const float DzEx = stencil_lds<2, AX>(E[0], sb, cell, S.M[2]);
       By[c] = By[c] + dt * (DxEz - DzEx);
-      const float DyEx = stencil_lds<1>(E[0], sb, cell, S.M[1]);
-      const float DxEy = stencil_lds<0>(E[1], sb, cell, S.M[0]);
+      const float DyEx = stencil_lds<1, AX>(E[0], sb, cell, S.M[1]);
+      const float DxEy = stencil_lds<0, AX>(E[1], sb, cell, S.M[0]);
       Bz[c] = Bz[c] + dt * (DyEx - DxEy);
+    };
+    if(active) {
+      if(full) update(std::false_type {});
+      else update(std::true_type {});
     }
     __syncthreads();
     base = base == 5 ? 0 : base + 1;
@@ -618,7 +640,7 @@ __global__ void __launch_bounds__(64) k_ghost_copy(Geo g, int nrows, float* F0, 
 // i), the workgroups after them the z layers of the other rows, six lanes a row.
 // Small worlds are bound by latency, also that of fetching the code: 64^3 took
 // 17 us with all components, the general case below and a workgroup per row in
-// one kernel, and the copy 5 us; @@FOLD@@
+// one kernel, and the copy 5 us; 5 us so (256^3: 50 us with the copy, 25 so).
 __global__ void __launch_bounds__(256) k_fold_copy(Geo g, int nrows, int copy, float* F0, float* F1, float* F2)
 {
   float* const F = blockIdx.y == 0 ? F0 : (blockIdx.y == 1 ? F1 : F2);
@@ -787,8 +809,17 @@ int launch_curl_b_stencil(rk_world* w, const int r0[3], const int r1[3], float d
   StencilM S;
   std::memcpy(S.M, w->stencil, sizeof(S.M));
   dim3 grid = region_grid(r);
-  grid.z = unsigned((r.r1[0] - r.r0[0] + SCH - 1) / SCH);
-  hipLaunchKernelGGL(k_curl_b_stencil, grid, dim3(BX, BY), 0, s, w->g, r, dt, S, w->E[0], w->E[1],
+  // long segments stage few planes twice; the launch still needs the three
+  // blocks per CU that fit
+  const int planes = r.r1[0] - r.r0[0];
+  int xseg = 32;
+  while(xseg > 4 && int64_t(grid.x) * grid.y * ((planes + xseg - 1) / xseg) < 768) xseg /= 2;
+  grid.z = unsigned((planes + xseg - 1) / xseg);
+  bool axial = true;
+  for(int a = 0; a < 3; ++a)
+    for(int n = 1; n < 3; ++n)
+      for(int col = 1; col < 5; ++col) axial = axial && S.M[a][n][col] == 0.0f;
+  hipLaunchKernelGGL(k_curl_b_stencil, grid, dim3(BX, BY), 0, s, w->g, r, dt, S, xseg, int(axial), w->E[0], w->E[1],
                      w->E[2], w->B[0], w->B[1], w->B[2]);
   RK_HIP(hipGetLastError());
   return RK_OK;
