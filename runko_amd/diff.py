@@ -85,8 +85,9 @@ class DiffBox:
 
     def _check(self, state):
         E, B, x, u = state
-        for t, shape in ((E, self._fshape), (B, self._fshape), (x, (3, self.np)), (u, (3, self.np))):
-            if tuple(t.shape) != shape or t.dtype != self.dtype or t.device != self.dev or not t.is_contiguous():
+        pshape = (3, self.np)
+        for t, shape in ((E, self._fshape), (B, self._fshape), (x, pshape), (u, pshape)):
+            if t.shape != shape or t.dtype != self.dtype or t.device != self.dev or not t.is_contiguous():
                 raise ValueError(f"DiffBox: expected a contiguous {self.dtype} tensor of shape {shape} on "
                                  f"{self.dev}, got {tuple(t.shape)} {t.dtype} {t.device}")
 
@@ -94,9 +95,9 @@ class DiffBox:
     def _struct(state):
         s = L.DiffState()
         for name, t in zip(("E", "B", "x", "u"), state):
-            arr = getattr(s, name)
-            for c in range(3):
-                arr[c] = t[c].data_ptr()
+            # three components of a contiguous tensor
+            p, step = t.data_ptr(), t.numel() // 3 * t.element_size()
+            getattr(s, name)[:] = (p, p + step, p + 2 * step)
         return s
 
     # ------------------------------------------------------------------ steps
@@ -105,7 +106,8 @@ class DiffBox:
         self._check(state)
         if out is None:
             out = self.empty_state()
-        self._check(out)
+        elif out is not state:
+            self._check(out)
         a, b = self._struct(state), self._struct(out)
         L.check(L.lib().rk_diff_step(self.h, ctypes.byref(a), ctypes.byref(b), _stream()))
         return out
@@ -116,7 +118,8 @@ class DiffBox:
         self._check(adj_out)
         if adj_in is None:
             adj_in = self.empty_state()
-        self._check(adj_in)
+        elif adj_in is not adj_out:
+            self._check(adj_in)
         a, b, c = self._struct(state), self._struct(adj_out), self._struct(adj_in)
         L.check(L.lib().rk_diff_step_adjoint(self.h, ctypes.byref(a), ctypes.byref(b), ctypes.byref(c), _stream()))
         return adj_in
@@ -279,24 +282,25 @@ class _Rollout(torch.autograd.Function):
     @staticmethod
     def forward(ctx, box, steps, every, E, B, x, u):
         levels = checkpoint_levels(every)
-        s = tuple(t.detach().contiguous().clone() for t in (E, B, x, u))
-        spare = box.empty_state()
-        ckpts = []
+        s = tuple(t.detach().clone(memory_format=torch.contiguous_format) for t in (E, B, x, u))
+        spare, ckpts = None, []
         for t in range(steps):
-            if t % levels[0] == 0:
-                ckpts.append(tuple(v.clone() for v in s))
-            box.step(s, spare)
-            s, spare = spare, s
+            # a checkpointed state is kept as it is, not copied
+            keep = t % levels[0] == 0
+            if keep:
+                ckpts.append(s)
+            new = box.step(s, spare)
+            s, spare = new, None if keep else s
         ctx.box, ctx.steps, ctx.levels, ctx.ckpts = box, steps, levels, ckpts
         return s
 
     @staticmethod
     def backward(ctx, gE, gB, gx, gu):
         box, steps, levels = ctx.box, ctx.steps, ctx.levels
-        ref = box.empty_state()
-        lam = tuple(torch.zeros_like(r) if g is None else g.detach().contiguous().clone()
-                    for g, r in zip((gE, gB, gx, gu), ref))
-        del ref
+        shapes = (box._fshape, box._fshape, (3, box.np), (3, box.np))
+        lam = tuple(torch.zeros(sh, dtype=box.dtype, device=box.dev) if g is None
+                    else g.detach().clone(memory_format=torch.contiguous_format)
+                    for g, sh in zip((gE, gB, gx, gu), shapes))
         k = levels[0]
         for seg in reversed(range(len(ctx.ckpts))):
             t0 = seg * k

@@ -43,7 +43,9 @@ def choose_brick(n_cells):
 
 
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    # the current stream's handle without a Stream object around it (about 5 us
+    # less per call of the library)
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
 
 
 def free_device_bytes(dev):
