@@ -297,10 +297,11 @@ class _Rollout(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gE, gB, gx, gu):
         box, steps, levels = ctx.box, ctx.steps, ctx.levels
-        shapes = (box._fshape, box._fshape, (3, box.np), (3, box.np))
-        lam = tuple(torch.zeros(sh, dtype=box.dtype, device=box.dev) if g is None
-                    else g.detach().clone(memory_format=torch.contiguous_format)
-                    for g, sh in zip((gE, gB, gx, gu), shapes))
+        grads = (gE, gB, gx, gu)
+        ref = box.empty_state() if any(g is None for g in grads) else grads
+        lam = tuple(torch.zeros_like(r) if g is None else g.detach().clone(memory_format=torch.contiguous_format)
+                    for g, r in zip(grads, ref))
+        del ref
         k = levels[0]
         for seg in reversed(range(len(ctx.ckpts))):
             t0 = seg * k
