@@ -299,6 +299,14 @@ int rk_move_bins(rk_world* w, int32_t s, int32_t n, const int32_t* bins, const i
 int rk_relayout(rk_world* w, int32_t s, const uint32_t* new_cap, void* tmp, int64_t tmp_bytes,
                 int64_t* new_start, void* stream);
 
+/* One tile's alive particles of species s in id order (equal ids in bin
+ * order) into device memory, asynchronously: what 0 positions, 1 momenta
+ * (float out[3][capacity]), 2 ids (uint64 out[capacity]); *count_dev their
+ * number.  For capacity <= 8192 (the tile's bin capacities) and at most 256
+ * bricks a tile. */
+int rk_tile_particles_by_id(rk_world* w, int32_t tile, int32_t s, int32_t what, int64_t capacity, uint64_t* count_dev,
+                            void* out, void* stream);
+
 /* Copies of one tile's alive particles of species s in bin order into caller
  * device buffers (capacity >= count); *count_out set synchronously. */
 int rk_tile_particle_count(rk_world* w, int32_t tile, int32_t s, int64_t* count_out, void* stream);

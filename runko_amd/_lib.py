@@ -74,6 +74,8 @@ _lib = None
 
 P3 = ctypes.c_void_p * 3
 
+READBACK_MAX, READBACK_BINS = 8192, 256  # limits of rk_tile_particles_by_id
+
 
 def lib():
     """Load the HIP library (raises if it was not built)."""
@@ -130,6 +132,7 @@ def lib():
     L.rk_relayout.argtypes = [vp, i32, vp, vp, i64, vp, vp]
     L.rk_tile_particle_count.argtypes = [vp, i32, i32, ctypes.POINTER(i64), vp]
     L.rk_tile_particles.argtypes = [vp, i32, i32, P3, P3, vp, i64, ctypes.POINTER(i64), vp]
+    L.rk_tile_particles_by_id.argtypes = [vp, i32, i32, i32, i64, vp, vp, vp]
     L.rk_outgoing.argtypes = [vp, P3, P3, vp, vp, vp, vp, i64, ctypes.POINTER(i64), vp]
     L.rk_energies.argtypes = [vp, i32, vp, vp]
     L.rk_energies_device.argtypes = [vp, i32, vp, vp]
@@ -173,7 +176,7 @@ EXPORTED = [
     "rk_profile_read", "rk_world_set_mailbox", "rk_world_set_current_staging", "rk_reflect_particles",
     "rk_apply_edge_bc", "rk_diff_create", "rk_diff_create_ensemble", "rk_diff_destroy", "rk_diff_step", "rk_diff_step_adjoint",
     "rk_diff_error_count", "rk_snapshot_fields", "rk_snapshot_spectra", "rk_interpolate_at",
-    "rk_world_set_schemes", "rk_push_half_b_comm", "rk_push_e_add_current_comm", "rk_exchange_current",
+    "rk_world_set_schemes", "rk_tile_particles_by_id", "rk_push_half_b_comm", "rk_push_e_add_current_comm", "rk_exchange_current",
 ]
 
 PROF_CATEGORIES = ["fused_particle_step", "push", "deposit", "pack", "append", "fdtd", "filter", "ghost", "other"]

@@ -850,6 +850,20 @@ int rk_tile_particles(rk_world* w, int32_t tile, int32_t s, float* const pos[3],
   return rc;
 }
 
+int rk_tile_particles_by_id(rk_world* w, int32_t tile, int32_t s, int32_t what, int64_t capacity, uint64_t* count_dev,
+                            void* out, void* stream)
+{
+  if(int rc = check_tile(w, tile)) return rc;
+  if(tile < 0) return fail(RK_EINVAL, "readback needs one tile");
+  if(s < 0 || s >= w->d.n_species) return fail(RK_EINVAL, "invalid species");
+  if(int rc = check_particles(w)) return rc;
+  if(what < 0 || what > 2) return fail(RK_EINVAL, "readback: positions, velocities or ids");
+  if(!count_dev || !out) return fail(RK_EINVAL, "null argument");
+  if(capacity < 0 || capacity > READBACK_MAX || w->g.bpt > READBACK_BINS)
+    return fail(RK_EINVAL, "readback by id: at most 8192 slots and 256 bricks a tile");
+  return launch_readback(w, tile, s, what, capacity, count_dev, out, S(stream));
+}
+
 int rk_outgoing(rk_world* w, float* const pos[3], float* const vel[3], uint64_t* id, int32_t* src_tile, int32_t* dir,
                 int32_t* species, int64_t capacity, int64_t* count_out, void* stream)
 {

@@ -267,6 +267,9 @@ int launch_move_bins(rk_world* w, int s, int n, const int32_t* bins, const int64
 int launch_filter_x3(rk_world* w, hipStream_t s);
 int relayout_species(rk_world* w, int s, const uint32_t* new_cap, void* tmp, int64_t tmp_bytes,
                      int64_t* new_start, hipStream_t st);
+constexpr int READBACK_BINS = 256;
+constexpr int64_t READBACK_MAX = 8192;
+int launch_readback(rk_world* w, int tile, int s, int what, int64_t capacity, uint64_t* count, void* out, hipStream_t st);
 int launch_gather_tile(rk_world* w, int tile, int s, float* const pos[3], float* const vel[3], uint64_t* id,
                        const int64_t* offsets_dev, hipStream_t st);
 int gauss_residual(rk_world* w, int passes, double* out, hipStream_t s);

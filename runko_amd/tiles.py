@@ -427,19 +427,26 @@ class PicTile(EmfTile):
         o = torch.sort(i, stable=True).indices
         return p[:, o], v[:, o], i[o]
 
+    def _read(self, s, what):
+        """Positions, velocities or ids (what = 0, 1, 2) on the host in id order."""
+        if s < 0 or s >= len(self._charges):
+            raise IndexError("particle type out of range")
+        torch.cuda.synchronize()
+        a = self._world.tile_particles_by_id(self._t, s, what)
+        if a is None:
+            a = self._particles(s)[what].cpu().numpy()
+        return a
+
     def get_positions(self, s):
-        p, _, _ = self._particles(s)
-        p = p.cpu().numpy()
+        p = self._read(s, 0)
         return (p[0].copy(), p[1].copy(), p[2].copy())
 
     def get_velocities(self, s):
-        _, v, _ = self._particles(s)
-        v = v.cpu().numpy()
+        v = self._read(s, 1)
         return (v[0].copy(), v[1].copy(), v[2].copy())
 
     def get_ids(self, s):
-        _, _, i = self._particles(s)
-        return i.cpu().numpy().view(np.uint64).copy()
+        return self._read(s, 2).view(np.uint64).copy()
 
     def number_of_species(self):
         return len(self._charges)

@@ -616,6 +616,25 @@ class World:
                                           ctypes.byref(got), _stream()))
         return pos[:, :n], vel[:, :n], ids[:n]
 
+    def tile_particles_by_id(self, t, s, what):
+        """Host copy of the tile's positions (what = 0) or momenta (1), float32
+        [3, n], or ids (2), uint64 [n], in id order; None where the tile has no
+        bins yet or is too large for the one-launch readback
+        (rk_tile_particles_by_id)."""
+        bpt = self.nbricks // self.ntiles
+        cap = int(self.pools[s].cap_h[t * bpt:(t + 1) * bpt].sum())
+        if cap == 0 or cap > L.READBACK_MAX or bpt > L.READBACK_BINS:
+            return None
+        size = 8 * cap if what == 2 else 12 * cap
+        buf = torch.empty((16 + size,), dtype=torch.uint8, device=self.dev)  # the count, then the data
+        p = buf.data_ptr()
+        L.check(L.lib().rk_tile_particles_by_id(self.h, int(t), int(s), what, cap, p, p + 16, _stream()))
+        h = buf.cpu().numpy()
+        n = int(h[:8].view(np.uint64)[0])
+        if what == 2:
+            return h[16:].view(np.uint64)[:n]
+        return h[16:].view(np.float32).reshape(3, cap)[:, :n]
+
     def outgoing(self):
         cap = self._mig_cap[0]
         pos = torch.empty((3, cap), dtype=torch.float32, device=self.dev)
