@@ -444,9 +444,12 @@ __global__ void __launch_bounds__(BX* BY)
 // (second) and starts the node one plane ahead (first).  Each sum thus takes
 // its taps in the order of filter_columns (x offset, then y, then z, from 0),
 // and a level's completed planes reach the next level through LDS (planes
-// double-buffered per level, one barrier per step).  The x segment is at
-// most F3XS planes and shorter on small worlds, so that the launch still has
-// a few workgroups per CU.
+// double-buffered per level, one barrier per step).  A workgroup takes one
+// component (blockIdx.z): the arithmetic of a step is then a third, and more
+// waves share a SIMD (42 registers for 88), which hides the steps' LDS latency:
+// 64^3 23 -> 14 us, 256^3 300 -> 230 us.  The x segment is at most F3XS planes
+// and shorter on small worlds, so that the launch still has a few workgroups
+// per CU.
 constexpr int F3Y = 8, F3Z = 32, F3T = 256, F3XS = 128;
 constexpr int F3IY = F3Y + 6, F3IZ = F3Z + 6, F3IN = F3IY * F3IZ, F3IM = (F3IN + F3T - 1) / F3T;
 
@@ -490,15 +493,16 @@ __global__ void __launch_bounds__(F3T)
   k_filter27_x3(Geo g, int xseg, const float* __restrict__ S0, const float* __restrict__ S1,
                 const float* __restrict__ S2, float* __restrict__ D0, float* __restrict__ D1, float* __restrict__ D2)
 {
-  __shared__ float In[2][3][F3IN];
-  __shared__ float L1[2][3][F3Level<1>::NP];
-  __shared__ float L2[2][3][F3Level<2>::NP];
+  __shared__ float In[2][F3IN];
+  __shared__ float L1[2][F3Level<1>::NP];
+  __shared__ float L2[2][F3Level<2>::NP];
   const int tid = int(threadIdx.x);
+  const int comp = int(blockIdx.z) % 3, seg = int(blockIdx.z) / 3;
+  const float* __restrict__ const S = comp == 0 ? S0 : (comp == 1 ? S1 : S2);
+  float* __restrict__ const D = comp == 0 ? D0 : (comp == 1 ? D1 : D2);
   const int z0 = HALO + int(blockIdx.x) * F3Z, y0 = HALO + int(blockIdx.y) * F3Y;
-  const int x0 = HALO + int(blockIdx.z) * xseg;
+  const int x0 = HALO + seg * xseg;
   const int xs = min(xseg, HALO + g.N[0] - x0);
-  const float* const S[3] = {S0, S1, S2};
-  float* const D[3] = {D0, D1, D2};
   // input plane q (0 .. xs+5) is haloed plane x0 - 3 + q; rows and columns
   // past the lattice (partial workgroups) read its last node and feed only
   // outputs that are not stored
@@ -513,26 +517,22 @@ __global__ void __launch_bounds__(F3T)
     ioff[m] = uint32_t(yy) * uint32_t(g.L[2]) + uint32_t(zz);
   }
   const uint32_t plane = uint32_t(g.L[1]) * uint32_t(g.L[2]);
-  float pre[3][F3IM];
+  float pre[F3IM];
   auto load = [&](int q) {
     const uint32_t base = uint32_t(x0 - HALO + q) * plane;
 #pragma unroll
-    for(int comp = 0; comp < 3; ++comp)
-#pragma unroll
-      for(int m = 0; m < F3IM; ++m)
-        if(iok[m]) pre[comp][m] = S[comp][base + ioff[m]];
+    for(int m = 0; m < F3IM; ++m)
+      if(iok[m]) pre[m] = S[base + ioff[m]];
   };
-  F3Chains c1[3][F3Level<1>::NM] = {}, c2[3][F3Level<2>::NM] = {}, c3[3][F3Level<3>::NM] = {};
+  F3Chains c1[F3Level<1>::NM] = {}, c2[F3Level<2>::NM] = {}, c3[F3Level<3>::NM] = {};
   const int nin = xs + 6;  // input planes
   load(0);
   for(int s = 0; s < xs + 9; ++s) {
     const int cur = s & 1, prev = cur ^ 1;
     if(s < nin) {
 #pragma unroll
-      for(int comp = 0; comp < 3; ++comp)
-#pragma unroll
-        for(int m = 0; m < F3IM; ++m)
-          if(iok[m]) In[cur][comp][tid + m * F3T] = pre[comp][m];
+      for(int m = 0; m < F3IM; ++m)
+        if(iok[m]) In[cur][tid + m * F3T] = pre[m];
       if(s + 1 < nin) load(s + 1);
     }
     // level 1 takes input plane s-1 and completes its node s-2 (input-relative index)
@@ -542,9 +542,7 @@ __global__ void __launch_bounds__(F3T)
         const int p = tid + m * F3T;
         if(p < F3Level<1>::NP) {
           const int py = p / F3Level<1>::WZ, pz = p - py * F3Level<1>::WZ;
-#pragma unroll
-          for(int comp = 0; comp < 3; ++comp)
-            L1[cur][comp][p] = f3_take<1>(In[prev][comp], py, pz, c1[comp][m]);
+          L1[cur][p] = f3_take<1>(In[prev], py, pz, c1[m]);
         }
       }
     }
@@ -555,9 +553,7 @@ __global__ void __launch_bounds__(F3T)
         const int p = tid + m * F3T;
         if(p < F3Level<2>::NP) {
           const int py = p / F3Level<2>::WZ, pz = p - py * F3Level<2>::WZ;
-#pragma unroll
-          for(int comp = 0; comp < 3; ++comp)
-            L2[cur][comp][p] = f3_take<2>(L1[prev][comp], py, pz, c2[comp][m]);
+          L2[cur][p] = f3_take<2>(L1[prev], py, pz, c2[m]);
         }
       }
     }
@@ -568,15 +564,9 @@ __global__ void __launch_bounds__(F3T)
         const int p = tid + m * F3T;
         if(p < F3Level<3>::NP) {
           const int py = p / F3Level<3>::WZ, pz = p - py * F3Level<3>::WZ;
-          float o[3];
-#pragma unroll
-          for(int comp = 0; comp < 3; ++comp) o[comp] = f3_take<3>(L2[prev][comp], py, pz, c3[comp][m]);
+          const float o = f3_take<3>(L2[prev], py, pz, c3[m]);
           const int y = y0 + py, z = z0 + pz;
-          if(s >= 9 && y < HALO + g.N[1] && z < HALO + g.N[2]) {
-            const uint32_t q = g.at(x0 - 9 + s, y, z);
-#pragma unroll
-            for(int comp = 0; comp < 3; ++comp) D[comp][q] = o[comp];
-          }
+          if(s >= 9 && y < HALO + g.N[1] && z < HALO + g.N[2]) D[g.at(x0 - 9 + s, y, z)] = o;
         }
       }
     }
@@ -871,9 +861,11 @@ int launch_filter_x3(rk_world* w, hipStream_t s)
   const Geo& g = w->g;
   const int64_t cols = int64_t((g.N[2] + F3Z - 1) / F3Z) * ((g.N[1] + F3Y - 1) / F3Y);
   int xseg = F3XS;
-  while(xseg > 4 && cols * ((g.N[0] + xseg - 1) / xseg) < 512) xseg /= 2;  // 2 workgroups per CU
+  // three workgroups per CU, one a component: fewer leave 128^3 at 69 us instead
+  // of 47, more, with their extra planes, 60 x 72 x 130 at 29 instead of 25
+  while(xseg > 2 && cols * ((g.N[0] + xseg - 1) / xseg) < 256) xseg /= 2;
   const dim3 grid(unsigned((g.N[2] + F3Z - 1) / F3Z), unsigned((g.N[1] + F3Y - 1) / F3Y),
-                  unsigned((g.N[0] + xseg - 1) / xseg));
+                  3 * unsigned((g.N[0] + xseg - 1) / xseg));
   hipLaunchKernelGGL(k_filter27_x3, grid, dim3(F3T), 0, s, g, xseg, w->J[0], w->J[1], w->J[2], w->Jf[0], w->Jf[1],
                      w->Jf[2]);
   RK_HIP(hipGetLastError());
