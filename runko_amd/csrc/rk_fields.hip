@@ -311,52 +311,44 @@ __global__ void __launch_bounds__(BX* BY)
 // c*P falls below the smallest normal float, 2^-126).
 // Same 27-tap filter, each lane sweeping a column of FCH outputs along x: the
 // 3x3 (y, z) neighbourhood of three consecutive x planes stays in registers,
-// so every input is loaded once per column instead of three times.  The
-// three components share the sweep, so a plane's 27 loads are in flight
-// together.  Each output still accumulates its 27 taps in layout_right order
-// from 0.
+// so every input is loaded once per column instead of three times.  A workgroup
+// takes one component (blockIdx.z): 45 registers instead of 105, twice the
+// waves to hide the loads' latency (64^3 13.8 -> 8.5 us, 256^3 184 -> 174 us).
+// Each output still accumulates its 27 taps in layout_right order from 0.
 constexpr int FCH = 8;
 
-__device__ inline void filter_columns(const Geo& g, const float* const (&S)[3], float* const (&D)[3], int i0, int i1,
+__device__ inline void filter_columns(const Geo& g, const float* __restrict__ S, float* __restrict__ D, int i0, int i1,
                                       int j, int k)
 {
   const uint32_t sj = uint32_t(g.L[2]);
-  float P[3][3][3][3];  // [component][plane i-1, i, i+1][b][c]
+  float P[3][3][3];  // [plane i-1, i, i+1][b][c]
   auto load = [&](int p, int i) {
     const uint32_t c0 = g.at(i, j, k);
 #pragma unroll
-    for(int q = 0; q < 3; ++q)
+    for(int b = 0; b < 3; ++b)
 #pragma unroll
-      for(int b = 0; b < 3; ++b)
-#pragma unroll
-        for(int cc = 0; cc < 3; ++cc) P[q][p][b][cc] = S[q][c0 + uint32_t(b - 1) * sj + uint32_t(cc - 1)];
+      for(int cc = 0; cc < 3; ++cc) P[p][b][cc] = S[c0 + uint32_t(b - 1) * sj + uint32_t(cc - 1)];
   };
   load(0, i0 - 1);
   load(1, i0);
   for(int i = i0; i < i1; ++i) {
     load(2, i + 1);
     const float w[3] = {1.0f, 2.0f, 1.0f};
-    const uint32_t c = g.at(i, j, k);
+    float acc = 0.0f;
 #pragma unroll
-    for(int q = 0; q < 3; ++q) {
-      float acc = 0.0f;
-#pragma unroll
-      for(int a = 0; a < 3; ++a)
-#pragma unroll
-        for(int b = 0; b < 3; ++b)
-#pragma unroll
-          for(int cc = 0; cc < 3; ++cc) acc = __builtin_fmaf((w[a] * w[b] * w[cc]) * (1.0f / 64.0f), P[q][a][b][cc], acc);
-      D[q][c] = acc;
-    }
-#pragma unroll
-    for(int q = 0; q < 3; ++q)
+    for(int a = 0; a < 3; ++a)
 #pragma unroll
       for(int b = 0; b < 3; ++b)
 #pragma unroll
-        for(int cc = 0; cc < 3; ++cc) {
-          P[q][0][b][cc] = P[q][1][b][cc];
-          P[q][1][b][cc] = P[q][2][b][cc];
-        }
+        for(int cc = 0; cc < 3; ++cc) acc = __builtin_fmaf((w[a] * w[b] * w[cc]) * (1.0f / 64.0f), P[a][b][cc], acc);
+    D[g.at(i, j, k)] = acc;
+#pragma unroll
+    for(int b = 0; b < 3; ++b)
+#pragma unroll
+      for(int cc = 0; cc < 3; ++cc) {
+        P[0][b][cc] = P[1][b][cc];
+        P[1][b][cc] = P[2][b][cc];
+      }
   }
 }
 
@@ -366,12 +358,11 @@ __global__ void __launch_bounds__(BX* BY)
 {
   const int k = r.r0[2] + int(blockIdx.x) * BX + int(threadIdx.x);
   const int j = r.r0[1] + int(blockIdx.y) * BY + int(threadIdx.y);
-  const int i0 = r.r0[0] + int(blockIdx.z) * FCH;
+  const int comp = int(blockIdx.z) % 3;
+  const int i0 = r.r0[0] + int(blockIdx.z) / 3 * FCH;
   const int i1 = min(i0 + FCH, r.r1[0]);
   if(k >= r.r1[2] || j >= r.r1[1]) return;
-  const float* const S[3] = {S0, S1, S2};
-  float* const D[3] = {D0, D1, D2};
-  filter_columns(g, S, D, i0, i1, j, k);
+  filter_columns(g, comp == 0 ? S0 : (comp == 1 ? S1 : S2), comp == 0 ? D0 : (comp == 1 ? D1 : D2), i0, i1, j, k);
 }
 
 // separable z, y, x passes (0.25, 0.5, 0.25), each output evaluated with the
@@ -379,7 +370,8 @@ __global__ void __launch_bounds__(BX* BY)
 // a column of FCH outputs along x; the z-then-y partial of a plane,
 //   T(p) = 0.25 Z(p, j-1) + 0.5 Z(p, j) + 0.25 Z(p, j+1),
 // depends on the plane alone, so each is computed once and reused by the
-// three outputs that take it.
+// three outputs that take it.  One component a workgroup (64^3 10.5 -> 8.1 us,
+// 256^3 173 us either way: memory).
 __device__ inline float sep_z(const float* __restrict__ S, uint32_t q)
 {
   return 0.25f * S[q - 1] + 0.5f * S[q] + 0.25f * S[q + 1];
@@ -393,26 +385,15 @@ __device__ inline float sep_zy(const Geo& g, const float* __restrict__ S, int i,
   return 0.25f * y0 + 0.5f * y1 + 0.25f * y2;
 }
 
-__device__ inline void sep_columns(const Geo& g, const float* const (&S)[3], float* const (&D)[3], int i0, int i1,
+__device__ inline void sep_columns(const Geo& g, const float* __restrict__ S, float* __restrict__ D, int i0, int i1,
                                    int j, int k)
 {
-  float t0[3], t1[3];
-#pragma unroll
-  for(int q = 0; q < 3; ++q) {
-    t0[q] = sep_zy(g, S[q], i0 - 1, j, k);
-    t1[q] = sep_zy(g, S[q], i0, j, k);
-  }
+  float t0 = sep_zy(g, S, i0 - 1, j, k), t1 = sep_zy(g, S, i0, j, k);
   for(int i = i0; i < i1; ++i) {
-    float t2[3];
-#pragma unroll
-    for(int q = 0; q < 3; ++q) t2[q] = sep_zy(g, S[q], i + 1, j, k);
-    const uint32_t c = g.at(i, j, k);
-#pragma unroll
-    for(int q = 0; q < 3; ++q) {
-      D[q][c] = 0.25f * t0[q] + 0.5f * t1[q] + 0.25f * t2[q];
-      t0[q] = t1[q];
-      t1[q] = t2[q];
-    }
+    const float t2 = sep_zy(g, S, i + 1, j, k);
+    D[g.at(i, j, k)] = 0.25f * t0 + 0.5f * t1 + 0.25f * t2;
+    t0 = t1;
+    t1 = t2;
   }
 }
 
@@ -423,12 +404,11 @@ __global__ void __launch_bounds__(BX* BY)
 {
   const int k = r.r0[2] + int(blockIdx.x) * BX + int(threadIdx.x);
   const int j = r.r0[1] + int(blockIdx.y) * BY + int(threadIdx.y);
-  const int i0 = r.r0[0] + int(blockIdx.z) * FCH;
+  const int comp = int(blockIdx.z) % 3;
+  const int i0 = r.r0[0] + int(blockIdx.z) / 3 * FCH;
   const int i1 = min(i0 + FCH, r.r1[0]);
   if(k >= r.r1[2] || j >= r.r1[1]) return;
-  const float* const S[3] = {S0, S1, S2};
-  float* const D[3] = {D0, D1, D2};
-  sep_columns(g, S, D, i0, i1, j, k);
+  sep_columns(g, comp == 0 ? S0 : (comp == 1 ? S1 : S2), comp == 0 ? D0 : (comp == 1 ? D1 : D2), i0, i1, j, k);
 }
 
 // Three binomial2 passes in one launch, for a periodic world whose J ghost
@@ -842,13 +822,13 @@ int launch_filter(rk_world* w, const int r0[3], const int r1[3], hipStream_t s)
   if(empty(r)) return RK_OK;
   if(w->d.current_filter == 0) {
     dim3 grid = region_grid(r);
-    grid.z = unsigned((r.r1[0] - r.r0[0] + FCH - 1) / FCH);
+    grid.z = 3 * unsigned((r.r1[0] - r.r0[0] + FCH - 1) / FCH);
     hipLaunchKernelGGL(k_filter27c, grid, dim3(BX, BY), 0, s, w->g, r, w->J[0], w->J[1], w->J[2], w->Jf[0],
                        w->Jf[1], w->Jf[2]);
   }
   else {
     dim3 grid = region_grid(r);
-    grid.z = unsigned((r.r1[0] - r.r0[0] + FCH - 1) / FCH);
+    grid.z = 3 * unsigned((r.r1[0] - r.r0[0] + FCH - 1) / FCH);
     hipLaunchKernelGGL(k_filter_sep, grid, dim3(BX, BY), 0, s, w->g, r, w->J[0], w->J[1], w->J[2], w->Jf[0],
                        w->Jf[1], w->Jf[2]);
   }
