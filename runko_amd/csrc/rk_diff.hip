@@ -213,13 +213,15 @@ __global__ void __launch_bounds__(DWG)
 // R binomial2 passes (yee_lattice_current_filter_binomial2.c++:23-76) of a
 // periodic box in one pass over memory: the passes are separable and commute,
 // so together they are (2R+1)-tap binomials along z, y and x.  A workgroup
-// owns FY x FZ columns of nodes and marches over xseg planes: each arriving
-// plane is staged in LDS with R nodes around the tile, summed along z (four
-// nodes a thread, which share their reads) and then along y (four nodes a
-// thread, a component per wave), and kept in registers for the 2R+1 sums along
-// x that take it; the next plane's loads are in flight meanwhile.  LDS reads
-// bound it: 23.6 us on 96^3 cells (66 us as three 27-tap launches).
-constexpr int FY = 8, FZ = 32;
+// owns FY x FZ columns of nodes of one component and marches over xseg planes:
+// each arriving plane is staged in LDS with R nodes around the tile, summed
+// along z (four nodes a thread, which share their reads) and then along y (four
+// nodes a thread, one wave), and kept in registers for the 2R+1 sums along x
+// that take it; the next plane's loads are in flight meanwhile.  LDS reads bound
+// it on large boxes: 22.3 us on 96^3 cells (66 us as three 27-tap launches); on
+// small ones the chain of a plane's two barriers does, shorter with a component
+// a workgroup than with all three in one of 256 threads: 16^3 12.7 -> 9.4 us.
+constexpr int FY = 8, FZ = 32, FT = 128;
 
 template<class T, int R>
 struct Taps {
@@ -245,20 +247,22 @@ __device__ inline T tap_sum(const T (&v)[N], int o)
 }
 
 template<class T, int R>
-__global__ void __launch_bounds__(FY* FZ)
+__global__ void __launch_bounds__(FT)
   k_dfilter(const DEnt<T>* __restrict__ tab, G3<T> out, G3<T> in, int tiles_z, int xseg)
 {
-  constexpr int NT = FY * FZ, IY = FY + 2 * R, IZ = FZ + 2 * R, NI = IY * IZ, NM = (NI + NT - 1) / NT;
-  constexpr int PZ = (IZ + 3) / 4 * 4, ZG = FZ / 4, TASKS = 3 * IY * ZG;
-  __shared__ alignas(32) T pl[2][3][IY * PZ];
-  __shared__ alignas(32) T zs[2][3][IY * FZ];
+  constexpr int IY = FY + 2 * R, IZ = FZ + 2 * R, NI = IY * IZ, NM = (NI + FT - 1) / FT;
+  constexpr int PZ = (IZ + 3) / 4 * 4, ZG = FZ / 4, TASKS = IY * ZG;
+  static_assert(TASKS <= FT && 2 * FZ <= FT && FY == 8, "a task a thread");
+  __shared__ alignas(32) T pl[2][IY * PZ];
+  __shared__ alignas(32) T zs[2][IY * FZ];
   const DEnt<T>& en = tab[blockIdx.z];
   const DBox<T>& b = en.b;
-  const int j0 = int(blockIdx.x) / tiles_z * FY, k0 = int(blockIdx.x) % tiles_z * FZ, i0 = int(blockIdx.y) * xseg;
+  const int comp = int(blockIdx.x) % 3, tile = int(blockIdx.x) / 3;
+  const int j0 = tile / tiles_z * FY, k0 = tile % tiles_z * FZ, i0 = int(blockIdx.y) * xseg;
   if(i0 >= b.n[0] || j0 >= b.n[1] || k0 >= b.n[2]) return;  // uniform over the workgroup
   const int i1 = min(i0 + xseg, b.n[0]);
-  in = sh(in, en.c0);
-  out = sh(out, en.c0);
+  const T* __restrict__ const src = (comp == 0 ? in.c[0] : (comp == 1 ? in.c[1] : in.c[2])) + en.c0;
+  T* __restrict__ const dst = (comp == 0 ? out.c[0] : (comp == 1 ? out.c[1] : out.c[2])) + en.c0;
   const int tid = int(threadIdx.x);
   auto wrapm = [](int i, int n) {
     while(i < 0) i += n;
@@ -268,44 +272,39 @@ __global__ void __launch_bounds__(FY* FZ)
   int off[NM], at[NM];
 #pragma unroll
   for(int m = 0; m < NM; ++m) {
-    const int e = min(tid + m * NT, NI - 1);  // (the last threads repeat the last node)
+    const int e = min(tid + m * FT, NI - 1);  // (the last threads repeat the last node)
     off[m] = wrapm(j0 - R + e / IZ, b.n[1]) * b.n[2] + wrapm(k0 - R + e % IZ, b.n[2]);
     at[m] = e / IZ * PZ + e % IZ;
   }
-  T pre[3][NM];
+  T pre[NM];
   auto load = [&](int i) {
-    const int64_t base = int64_t(wrapm(i, b.n[0])) * b.n[1] * b.n[2];
+    const T* const plane = src + int64_t(wrapm(i, b.n[0])) * b.n[1] * b.n[2];
 #pragma unroll
-    for(int c = 0; c < 3; ++c)
-#pragma unroll
-      for(int m = 0; m < NM; ++m) pre[c][m] = in.c[c][base + off[m]];
+    for(int m = 0; m < NM; ++m) pre[m] = plane[off[m]];
   };
   T ring[4][2 * R + 1] = {};
-  const int yc = tid / 64, ty = tid % 64 / FZ * 4, tz = tid % FZ;  // the y and x sums: threads 0..191
-  T* const dst = yc == 0 ? out.c[0] : (yc == 1 ? out.c[1] : out.c[2]);
+  const int ty = tid / FZ * 4, tz = tid % FZ;  // the y and x sums: threads 0..63
   load(i0 - R);
   for(int i = i0 - R; i < i1 + R; ++i) {
     const int cur = i & 1;
 #pragma unroll
-    for(int c = 0; c < 3; ++c)
-#pragma unroll
-      for(int m = 0; m < NM; ++m) pl[cur][c][at[m]] = pre[c][m];
+    for(int m = 0; m < NM; ++m) pl[cur][at[m]] = pre[m];
     if(i + 1 < i1 + R) load(i + 1);
     __syncthreads();
-    for(int q = tid; q < TASKS; q += NT) {
-      const int c = q / (IY * ZG), row = q / ZG % IY, zg = q % ZG;
-      const T* p = &pl[cur][c][row * PZ + zg * 4];
+    if(tid < TASKS) {
+      const int row = tid / ZG, zg = tid % ZG;
+      const T* p = &pl[cur][row * PZ + zg * 4];
       T v[4 + 2 * R];
 #pragma unroll
       for(int k = 0; k < 4 + 2 * R; ++k) v[k] = p[k];
 #pragma unroll
-      for(int k = 0; k < 4; ++k) zs[cur][c][row * FZ + zg * 4 + k] = tap_sum<T, R>(v, k);
+      for(int k = 0; k < 4; ++k) zs[cur][row * FZ + zg * 4 + k] = tap_sum<T, R>(v, k);
     }
     __syncthreads();
-    if(tid < 192) {
+    if(tid < 2 * FZ) {
       T v[4 + 2 * R];
 #pragma unroll
-      for(int k = 0; k < 4 + 2 * R; ++k) v[k] = zs[cur][yc][(ty + k) * FZ + tz];
+      for(int k = 0; k < 4 + 2 * R; ++k) v[k] = zs[cur][(ty + k) * FZ + tz];
 #pragma unroll
       for(int y = 0; y < 4; ++y) {
 #pragma unroll
@@ -1480,11 +1479,11 @@ int filter_passes(const DiffImpl& h, const DEnt<T>* b, G3<T>& f, hipStream_t st)
   const int tz = (h.nmax[2] + FZ - 1) / FZ, cols = tz * ((h.nmax[1] + FY - 1) / FY);
   int xseg = h.nmax[0];
   while(xseg > 2 && int64_t(cols) * ((h.nmax[0] + xseg - 1) / xseg) * int64_t(h.boxes.size()) < 512) xseg = (xseg + 1) / 2;
-  const dim3 grid(unsigned(cols), unsigned((h.nmax[0] + xseg - 1) / xseg), unsigned(h.boxes.size()));
+  const dim3 grid(3 * unsigned(cols), unsigned((h.nmax[0] + xseg - 1) / xseg), unsigned(h.boxes.size()));
   for(int left = h.d.filter_passes; left > 0;) {
     const int r = std::min(left, 3);
     const G3<T> out = g3s<T>(h, o);
-    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(FY * FZ), 0, st, b, out, f, tz, xseg); };
+    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(FT), 0, st, b, out, f, tz, xseg); };
     r == 3 ? go(k_dfilter<T, 3>) : (r == 2 ? go(k_dfilter<T, 2>) : go(k_dfilter<T, 1>));
     RK_HIP(hipGetLastError());
     f = out;
