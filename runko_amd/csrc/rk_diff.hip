@@ -141,19 +141,40 @@ __device__ inline void atomic_add(T* p, T v)
 // out = in + dt * curlE(E)   (push_b_fdtd2 order; out may alias in); clears
 // the planar field Z when it is given
 template<class T>
-__global__ void __launch_bounds__(DWG)
-  k_dcurl_b(const DEnt<T>* __restrict__ tab, G3<T> out, G3<T> in, G3<T> E, T dt, G3<T> Z)
+struct CurlB {
+  G3<T> out, in, E;
+  T dt;
+  G3<T> Z;
+};
+
+// The grid of a per-box launch (grid_of, block_of) as part of a launch of 1D
+// workgroups of DWG threads.
+struct BoxGrid {
+  int gx, gy, gz, bx, by;
+  __host__ __device__ int blocks() const { return gx * gy * gz; }
+};
+struct BoxPlace {
+  int z, i, j, tx;
+  bool ok;
+};
+__device__ inline BoxPlace place(const BoxGrid& g, int blk)
 {
-  const DEnt<T>& en = tab[blockIdx.z];
+  const int tid = int(threadIdx.x), ty = tid / g.bx, x = blk % g.gx, q = blk / g.gx;
+  return BoxPlace {q / g.gy, q % g.gy, x * g.by + ty, tid - ty * g.bx, ty < g.by};
+}
+
+// the nodes (i, j, k), k = tx, tx + bx, ..., of a box
+template<class T>
+__device__ inline void curl_b_row(const DEnt<T>& en, const CurlB<T>& u, int i, int j, int tx, int bx)
+{
   const DBox<T>& b = en.b;
-  const int j = int(blockIdx.x * blockDim.y + threadIdx.y), i = int(blockIdx.y);
   if(j >= b.n[1] || i >= b.n[0]) return;
-  out = sh(out, en.c0);
-  in = sh(in, en.c0);
-  E = sh(E, en.c0);
+  const G3<T> out = sh(u.out, en.c0);
+  const G3<T> in = sh(u.in, en.c0);
+  const G3<T> E = sh(u.E, en.c0);
   const int n0 = b.n[0], n1 = b.n[1], n2 = b.n[2];
   const int ip = wrap1(i + 1, n0), jp = wrap1(j + 1, n1);
-  for(int k = int(threadIdx.x); k < n2; k += int(blockDim.x)) {
+  for(int k = tx; k < n2; k += bx) {
     const int kp = wrap1(k + 1, n2);
     const int64_t c = cidx(b.n, i, j, k);
     const T DkEy = E.c[1][cidx(b.n, i, j, kp)] - E.c[1][c];
@@ -162,13 +183,20 @@ __global__ void __launch_bounds__(DWG)
     const T DkEx = E.c[0][cidx(b.n, i, j, kp)] - E.c[0][c];
     const T DjEx = E.c[0][cidx(b.n, i, jp, k)] - E.c[0][c];
     const T DiEy = E.c[1][cidx(b.n, ip, j, k)] - E.c[1][c];
-    out.c[0][c] = in.c[0][c] + dt * (DkEy - DjEz);
-    out.c[1][c] = in.c[1][c] + dt * (DiEz - DkEx);
-    out.c[2][c] = in.c[2][c] + dt * (DjEx - DiEy);
-    if(Z.c[0])
+    out.c[0][c] = in.c[0][c] + u.dt * (DkEy - DjEz);
+    out.c[1][c] = in.c[1][c] + u.dt * (DiEz - DkEx);
+    out.c[2][c] = in.c[2][c] + u.dt * (DjEx - DiEy);
+    if(u.Z.c[0])
 #pragma unroll
-      for(int q = 0; q < 3; ++q) Z.c[q][en.c0 + c] = T(0);
+      for(int q = 0; q < 3; ++q) u.Z.c[q][en.c0 + c] = T(0);
   }
+}
+
+template<class T>
+__global__ void __launch_bounds__(DWG) k_dcurl_b(const DEnt<T>* __restrict__ tab, CurlB<T> u)
+{
+  curl_b_row(tab[blockIdx.z], u, int(blockIdx.y), int(blockIdx.x * blockDim.y + threadIdx.y), int(threadIdx.x),
+             int(blockDim.x));
 }
 
 // out = in + dt * curlB(B), then out -= J when J is given (push_e_fdtd2 +
@@ -410,18 +438,16 @@ __device__ inline void sum_windows(const DEnt<T>& en, const Cov& ci, const Cov& 
 // lambda_E += the bricks' windows of E adjoints (components 0..2 of mst),
 // lambda_B1 = lambda_B2 + their windows of B adjoints (3..5)
 template<class T, int BR>
-__global__ void __launch_bounds__(DWG)
-  k_dmgather(const DEnt<T>* __restrict__ tab, G3<T> LE, G3<T> LB, G3<T> LBout, const T* __restrict__ mst)
+__device__ inline void mgather_row(const DEnt<T>& en, G3<T> LE, G3<T> LB, G3<T> LBout, const T* __restrict__ mst, int i,
+                                   int j, int tx, int bx)
 {
   constexpr int W = BR + 2, V = W * W * W;
-  const DEnt<T>& en = tab[blockIdx.z];
   const DBox<T>& b = en.b;
-  const int j = int(blockIdx.x * blockDim.y + threadIdx.y), i = int(blockIdx.y);
   if(j >= b.n[1] || i >= b.n[0]) return;
   mst += en.k0 * (6 * V);
   const Cov ci = covers<1, 1>(en.ax[0], i);
   const Cov cj = covers<1, 1>(en.ax[1], j);
-  for(int k = int(threadIdx.x); k < b.n[2]; k += int(blockDim.x)) {
+  for(int k = tx; k < b.n[2]; k += bx) {
     const Cov ck = covers<1, 1>(en.ax[2], k);
     T s[6];
     sum_windows<T, 6, W>(en, ci, cj, ck, mst, s);
@@ -434,23 +460,28 @@ __global__ void __launch_bounds__(DWG)
   }
 }
 
+template<class T, int BR>
+__global__ void __launch_bounds__(DWG)
+  k_dmgather(const DEnt<T>* __restrict__ tab, G3<T> LE, G3<T> LB, G3<T> LBout, const T* __restrict__ mst)
+{
+  mgather_row<T, BR>(tab[blockIdx.z], LE, LB, LBout, mst, int(blockIdx.y), int(blockIdx.x * blockDim.y + threadIdx.y),
+                     int(threadIdx.x), int(blockDim.x));
+}
+
 // J += the bricks' current windows (jst, three components per brick).  J was
 // cleared before the particle step; it holds only contributions that missed
 // their brick's window.
 template<class T, int BR>
-__global__ void __launch_bounds__(DWG)
-  k_djgather(const DEnt<T>* __restrict__ tab, G3<T> J, const T* __restrict__ jst)
+__device__ inline void jgather_row(const DEnt<T>& en, G3<T> J, const T* __restrict__ jst, int i, int j, int tx, int bx)
 {
   constexpr int D = BR + 3, V = D * D * D;
-  const DEnt<T>& en = tab[blockIdx.z];
   const DBox<T>& b = en.b;
-  const int j = int(blockIdx.x * blockDim.y + threadIdx.y), i = int(blockIdx.y);
   if(j >= b.n[1] || i >= b.n[0]) return;
   J = sh(J, en.c0);
   jst += en.k0 * (3 * V);
   const Cov ci = covers<1, 2>(en.ax[0], i);
   const Cov cj = covers<1, 2>(en.ax[1], j);
-  for(int k = int(threadIdx.x); k < b.n[2]; k += int(blockDim.x)) {
+  for(int k = tx; k < b.n[2]; k += bx) {
     const Cov ck = covers<1, 2>(en.ax[2], k);
     T s[3];
     sum_windows<T, 3, D>(en, ci, cj, ck, jst, s);
@@ -458,6 +489,14 @@ __global__ void __launch_bounds__(DWG)
 #pragma unroll
     for(int q = 0; q < 3; ++q) J.c[q][c] += s[q];
   }
+}
+
+template<class T, int BR>
+__global__ void __launch_bounds__(DWG)
+  k_djgather(const DEnt<T>* __restrict__ tab, G3<T> J, const T* __restrict__ jst)
+{
+  jgather_row<T, BR>(tab[blockIdx.z], J, jst, int(blockIdx.y), int(blockIdx.x * blockDim.y + threadIdx.y),
+                     int(threadIdx.x), int(blockDim.x));
 }
 
 // ---------------------------------------------------------------- particles
@@ -647,17 +686,17 @@ __device__ inline int base_cell(T x, T& d)
 __device__ inline int wrap2(int i, int n) { return wrap1(wrap1(i, n), n); }
 
 template<class T, int K, bool ADJ>
-__global__ void __launch_bounds__(1024)
-  k_dbin(const DEnt<T>* __restrict__ tab, const uint16_t* __restrict__ pmap, G3<T> x, G3<T> u, G3<T> lx, G3<T> lu,
+__device__ __forceinline__ void
+bin_block(int block, const DEnt<T>* __restrict__ tab, const uint16_t* __restrict__ pmap, G3<T> x, G3<T> u, G3<T> lx, G3<T> lu,
          uint32_t* __restrict__ rows, uint16_t* __restrict__ slot, Rec<T>* __restrict__ A, Rec<T>* __restrict__ B,
          unsigned long long* err)
 {
   extern __shared__ uint32_t hist[];  // two 16-bit counters per word: groups, then out-of-box particles
   __shared__ uint32_t wsum[16];
-  const DEnt<T>& en = tab[pmap[blockIdx.x]];
+  const DEnt<T>& en = tab[pmap[block]];
   const DBox<T>& b = en.b;
   const int nt = int(blockDim.x), tid = int(threadIdx.x);
-  const int64_t blk = int64_t(blockIdx.x) - en.pb0, P = int64_t(nt) * K;
+  const int64_t blk = int64_t(block) - en.pb0, P = int64_t(nt) * K;
   const int64_t np = b.off[b.nsp], p0 = blk * P;
   const int nw = en.rowlen;
   for(int w = tid; w < nw; w += nt) hist[w] = 0;
@@ -760,14 +799,23 @@ __global__ void __launch_bounds__(1024)
   }
 }
 
-template<class T, int K>
+template<class T, int K, bool ADJ>
 __global__ void __launch_bounds__(1024)
-  k_dunsort(const DEnt<T>* __restrict__ tab, const uint16_t* __restrict__ pmap, const uint16_t* __restrict__ slot,
+  k_dbin(const DEnt<T>* __restrict__ tab, const uint16_t* __restrict__ pmap, G3<T> x, G3<T> u, G3<T> lx, G3<T> lu,
+         uint32_t* __restrict__ rows, uint16_t* __restrict__ slot, Rec<T>* __restrict__ A, Rec<T>* __restrict__ B,
+         unsigned long long* err)
+{
+  bin_block<T, K, ADJ>(int(blockIdx.x), tab, pmap, x, u, lx, lu, rows, slot, A, B, err);
+}
+
+template<class T, int K>
+__device__ __forceinline__ void
+unsort_block(int block, const DEnt<T>* __restrict__ tab, const uint16_t* __restrict__ pmap, const uint16_t* __restrict__ slot,
             const Rec<T>* __restrict__ A, G3<T> x, G3<T> u)
 {
-  const DEnt<T>& en = tab[pmap[blockIdx.x]];
+  const DEnt<T>& en = tab[pmap[block]];
   const int nt = int(blockDim.x);
-  const int64_t np = en.b.off[en.b.nsp], p0 = (int64_t(blockIdx.x) - en.pb0) * nt * K;
+  const int64_t np = en.b.off[en.b.nsp], p0 = (int64_t(block) - en.pb0) * nt * K;
   constexpr int KC = K < 4 ? K : 4;
 #pragma unroll
   for(int k0 = 0; k0 < K; k0 += KC) {
@@ -786,6 +834,56 @@ __global__ void __launch_bounds__(1024)
           u.c[a][q[k]] = r[k].v[3 + a];
         }
   }
+}
+
+template<class T, int K>
+__global__ void __launch_bounds__(1024)
+  k_dunsort(const DEnt<T>* __restrict__ tab, const uint16_t* __restrict__ pmap, const uint16_t* __restrict__ slot,
+            const Rec<T>* __restrict__ A, G3<T> x, G3<T> u)
+{
+  unsort_block<T, K>(int(blockIdx.x), tab, pmap, slot, A, x, u);
+}
+
+// Small boxes (a particle a thread in the particle blocks): a launch costs
+// about 4 us whatever it does, so what needs nothing of each other shares one.
+// Before the bricks' step, the particles' bins and the curls of the fields; a
+// second curl (the adjoint's) when c2.out is given.  16^3 box, 16384 particles: six
+// launches a step instead of eight (adjoint: of nine), eight steps and their
+// gradient 1.02 -> 0.87 ms.
+template<class T, bool ADJ>
+__global__ void __launch_bounds__(DWG)
+  k_dprep(const DEnt<T>* __restrict__ tab, const uint16_t* __restrict__ pmap, G3<T> x, G3<T> u, G3<T> lx, G3<T> lu,
+          uint32_t* __restrict__ rows, uint16_t* __restrict__ slot, Rec<T>* __restrict__ A, Rec<T>* __restrict__ B,
+          unsigned long long* err, int pblocks, BoxGrid bg, CurlB<T> c1, CurlB<T> c2)
+{
+  int blk = int(blockIdx.x);
+  if(blk < pblocks) {
+    bin_block<T, 1, ADJ>(blk, tab, pmap, x, u, lx, lu, rows, slot, A, B, err);
+    return;
+  }
+  blk -= pblocks;
+  const bool second = blk >= bg.blocks();
+  const BoxPlace pl = place(bg, second ? blk - bg.blocks() : blk);
+  if(pl.ok) curl_b_row(tab[pl.z], second ? c2 : c1, pl.i, pl.j, pl.tx, bg.bx);
+}
+
+// After it, the particles back into their order and the gather of the bricks'
+// windows (the current's, or the adjoint's node means).
+template<class T, int BR, bool ADJ>
+__global__ void __launch_bounds__(DWG)
+  k_dfinish(const DEnt<T>* __restrict__ tab, const uint16_t* __restrict__ pmap, const uint16_t* __restrict__ slot,
+            const Rec<T>* __restrict__ A, G3<T> x, G3<T> u, int pblocks, BoxGrid bg, G3<T> F, G3<T> LB, G3<T> LBout,
+            const T* __restrict__ st)
+{
+  const int blk = int(blockIdx.x);
+  if(blk < pblocks) {
+    unsort_block<T, 1>(blk, tab, pmap, slot, A, x, u);
+    return;
+  }
+  const BoxPlace pl = place(bg, blk - pblocks);
+  if(!pl.ok) return;
+  if constexpr(ADJ) mgather_row<T, BR>(tab[pl.z], F, LB, LBout, st, pl.i, pl.j, pl.tx, bg.bx);
+  else jgather_row<T, BR>(tab[pl.z], F, st, pl.i, pl.j, pl.tx, bg.bx);
 }
 
 // one brick of a box
@@ -1520,6 +1618,42 @@ int unsort_particles(const DiffImpl& h, int which, G3<T> x, G3<T> u, hipStream_t
   return RK_OK;
 }
 
+inline BoxGrid box_grid(const DiffImpl& h)
+{
+  const dim3 g = grid_of(h), b = block_of(h);
+  return BoxGrid {int(g.x), int(g.y), int(g.z), int(b.x), int(b.y)};
+}
+
+// Launches are merged where they bound the step: particle blocks of DWG threads
+// with a particle each (up to 2^17 particles) and up to 2^18 cells, beyond which
+// the curls' rows (a workgroup of DWG threads however short) outweigh a launch.
+inline bool merged(const DiffImpl& h)
+{
+  return h.np > 0 && h.bin_k == 1 && h.bin_threads == DWG && h.ncell <= (int64_t(1) << 18);
+}
+
+// the bins of the particles, and before them the curls (c2: if c2.out is given)
+template<class T, bool ADJ>
+int prepare(const DiffImpl& h, G3<T> x, G3<T> u, G3<T> lx, G3<T> lu, const CurlB<T>& c1, const CurlB<T>& c2, hipStream_t st)
+{
+  const bool two = c2.out.c[0] != nullptr;
+  if(merged(h)) {
+    const BoxGrid bg = box_grid(h);
+    hipLaunchKernelGGL((k_dprep<T, ADJ>), dim3(unsigned(h.pblocks + (two ? 2 : 1) * bg.blocks())), dim3(DWG),
+                       sizeof(uint32_t) * size_t(h.rowlen_max), st, table<T>(h), h.pmap, x, u, lx, lu, h.rows, h.slot,
+                       static_cast<Rec<T>*>(h.recs[0]), static_cast<Rec<T>*>(h.recs[1]), h.err, int(h.pblocks), bg, c1, c2);
+    RK_HIP(hipGetLastError());
+    return RK_OK;
+  }
+  hipLaunchKernelGGL(k_dcurl_b<T>, grid_of(h), block_of(h), 0, st, table<T>(h), c1);
+  RK_HIP(hipGetLastError());
+  if(two) {
+    hipLaunchKernelGGL(k_dcurl_b<T>, grid_of(h), block_of(h), 0, st, table<T>(h), c2);
+    RK_HIP(hipGetLastError());
+  }
+  return h.np > 0 ? bin_particles<T, ADJ>(h, x, u, lx, lu, st) : RK_OK;
+}
+
 template<class T, int BR>
 int step_t(DiffImpl& h, const rk_diff_state* in, rk_diff_state* out, hipStream_t st)
 {
@@ -1529,23 +1663,30 @@ int step_t(DiffImpl& h, const rk_diff_state* in, rk_diff_state* out, hipStream_t
   const G3<T> E = g3<T>(in->E), B = g3<T>(in->B), B1 = g3s<T>(h, S_B1), J = g3s<T>(h, S_J);
   const int64_t P = int64_t(h.bin_threads) * h.bin_k;
   // B1 = B + cfl/2 curlE(E); J = 0
-  hipLaunchKernelGGL(k_dcurl_b<T>, grid_of(h), block_of(h), 0, st, b, B1, B, E, half, J);
-  RK_HIP(hipGetLastError());
+  if(int rc = prepare<T, false>(h, g3<T>(in->x), g3<T>(in->u), none, none, {B1, B, E, half, J}, {none, none, none, half, none}, st))
+    return rc;
   if(h.np > 0) {
-    if(int rc = bin_particles<T, false>(h, g3<T>(in->x), g3<T>(in->u), none, none, st)) return rc;
     constexpr int NT = brick_threads(BR);
     T* jst = static_cast<T*>(h.stage);
     hipLaunchKernelGGL((k_dstep<T, BR, NT>), dim3(unsigned(h.nbricks)), dim3(NT), 0, st, b, h.kmap, E, B1, h.rows, P,
                        static_cast<const Rec<T>*>(h.recs[0]), static_cast<Rec<T>*>(h.recs[h.grouped]), jst, J);
     RK_HIP(hipGetLastError());
-    hipLaunchKernelGGL((k_djgather<T, BR>), grid_of(h), block_of(h), 0, st, b, J, jst);
-    RK_HIP(hipGetLastError());
-    if(int rc = unsort_particles<T>(h, h.grouped, g3<T>(out->x), g3<T>(out->u), st)) return rc;
+    if(merged(h)) {
+      const BoxGrid bg = box_grid(h);
+      hipLaunchKernelGGL((k_dfinish<T, BR, false>), dim3(unsigned(h.pblocks + bg.blocks())), dim3(DWG), 0, st, b, h.pmap,
+                         h.slot, static_cast<const Rec<T>*>(h.recs[h.grouped]), g3<T>(out->x), g3<T>(out->u),
+                         int(h.pblocks), bg, J, none, none, jst);
+      RK_HIP(hipGetLastError());
+    } else {
+      hipLaunchKernelGGL((k_djgather<T, BR>), grid_of(h), block_of(h), 0, st, b, J, jst);
+      RK_HIP(hipGetLastError());
+      if(int rc = unsort_particles<T>(h, h.grouped, g3<T>(out->x), g3<T>(out->u), st)) return rc;
+    }
   }
   G3<T> jf = J;
   if(int rc = filter_passes<T>(h, b, jf, st)) return rc;
   // B2 = B1 + cfl/2 curlE(E), written to out.B (E is still the input E)
-  hipLaunchKernelGGL(k_dcurl_b<T>, grid_of(h), block_of(h), 0, st, b, g3<T>(out->B), B1, E, half, none);
+  hipLaunchKernelGGL(k_dcurl_b<T>, grid_of(h), block_of(h), 0, st, b, CurlB<T> {g3<T>(out->B), B1, E, half, none});
   RK_HIP(hipGetLastError());
   // E' = E + cfl curlB(B2) - Jf
   hipLaunchKernelGGL(k_dcurl_e<T>, grid_of(h), block_of(h), 0, st, b, g3<T>(out->E), E, g3<T>(out->B), full, jf);
@@ -1562,12 +1703,11 @@ int adjoint_t(DiffImpl& h, const rk_diff_state* in, const rk_diff_state* ao, rk_
   const G3<T> E = g3<T>(in->E), B = g3<T>(in->B), B1 = g3s<T>(h, S_B1);
   const G3<T> LEo = g3<T>(ao->E), LBo = g3<T>(ao->B), LB2 = g3s<T>(h, S_LB2), LE = g3s<T>(h, S_LE);
   const int64_t P = int64_t(h.bin_threads) * h.bin_k;
-  // forward B1
-  hipLaunchKernelGGL(k_dcurl_b<T>, grid_of(h), block_of(h), 0, st, b, B1, B, E, half, none);
-  RK_HIP(hipGetLastError());
+  // forward B1, and
   // E' = E + cfl curlB(B2) - Jf:  lambda_B2 = LB' + cfl curlB^T(LE') = LB' - cfl curlE(LE')
-  hipLaunchKernelGGL(k_dcurl_b<T>, grid_of(h), block_of(h), 0, st, b, LB2, LBo, LEo, T(-full), none);
-  RK_HIP(hipGetLastError());
+  if(int rc = prepare<T, true>(h, g3<T>(in->x), g3<T>(in->u), g3<T>(ao->x), g3<T>(ao->u), {B1, B, E, half, none},
+                               {LB2, LBo, LEo, T(-full), none}, st))
+    return rc;
   // B2 = B1 + cfl/2 curlE(E):  lambda_E = LE' + cfl/2 curlE^T(LB2) = LE' - cfl/2 curlB(LB2)
   hipLaunchKernelGGL(k_dcurl_e<T>, grid_of(h), block_of(h), 0, st, b, LE, LEo, LB2, T(-half), none);
   RK_HIP(hipGetLastError());
@@ -1576,17 +1716,24 @@ int adjoint_t(DiffImpl& h, const rk_diff_state* in, const rk_diff_state* ao, rk_
     // lambda_J = -F^P(LE')
     G3<T> lj = LEo;
     if(int rc = filter_passes<T>(h, b, lj, st)) return rc;
-    if(int rc = bin_particles<T, true>(h, g3<T>(in->x), g3<T>(in->u), g3<T>(ao->x), g3<T>(ao->u), st)) return rc;
     constexpr int NT = brick_threads(BR);
     T* mst = static_cast<T*>(h.stage);
     hipLaunchKernelGGL((k_dadj<T, BR, NT>), dim3(unsigned(h.nbricks)), dim3(NT), 0, st, b, h.kmap, E, B1, lj, h.rows, P,
                        static_cast<const Rec<T>*>(h.recs[0]), static_cast<Rec<T>*>(h.recs[1]), mst);
     RK_HIP(hipGetLastError());
-    if(int rc = unsort_particles<T>(h, 1, g3<T>(ai->x), g3<T>(ai->u), st)) return rc;
     // node-mean adjoints: lambda_E += NM_E^T(ME), lambda_B = lambda_B1 = LB2 + NM_B^T(MB)
     LB1 = g3<T>(ai->B);
-    hipLaunchKernelGGL((k_dmgather<T, BR>), grid_of(h), block_of(h), 0, st, b, LE, LB2, LB1, mst);
-    RK_HIP(hipGetLastError());
+    if(merged(h)) {
+      const BoxGrid bg = box_grid(h);
+      hipLaunchKernelGGL((k_dfinish<T, BR, true>), dim3(unsigned(h.pblocks + bg.blocks())), dim3(DWG), 0, st, b, h.pmap,
+                         h.slot, static_cast<const Rec<T>*>(h.recs[1]), g3<T>(ai->x), g3<T>(ai->u), int(h.pblocks), bg, LE,
+                         LB2, LB1, mst);
+      RK_HIP(hipGetLastError());
+    } else {
+      if(int rc = unsort_particles<T>(h, 1, g3<T>(ai->x), g3<T>(ai->u), st)) return rc;
+      hipLaunchKernelGGL((k_dmgather<T, BR>), grid_of(h), block_of(h), 0, st, b, LE, LB2, LB1, mst);
+      RK_HIP(hipGetLastError());
+    }
   } else {
     for(int c = 0; c < 3; ++c)
       RK_HIP(hipMemcpyAsync(ai->B[c], LB2.c[c], h.vb * size_t(h.ncell), hipMemcpyDeviceToDevice, st));
