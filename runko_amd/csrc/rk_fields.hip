@@ -48,11 +48,17 @@ bool ghosts_in_pass(const Geo& g)
 }
 
 __device__ inline int ghost_step(int c, int N) { return c < 2 * HALO ? N : (c >= N ? -N : 0); }
+// the step along axis 0 or 1 as an offset in the lattice (modulo 2^32, as its indices)
+__device__ inline int ghost_row(const Geo& g, int c, int axis)
+{
+  const uint32_t row = axis == 0 ? uint32_t(g.L[1]) * uint32_t(g.L[2]) : uint32_t(g.L[2]);
+  return int(uint32_t(ghost_step(c, g.N[axis])) * row);
+}
 
 __device__ inline void put_ghosts(const Geo& g, int i, int j, int k, uint32_t c, float* F0, float* F1, float* F2,
                                   float v0, float v1, float v2)
 {
-  const int d0 = ghost_step(i, g.N[0]) * g.L[1] * g.L[2], d1 = ghost_step(j, g.N[1]) * g.L[2];
+  const int d0 = ghost_row(g, i, 0), d1 = ghost_row(g, j, 1);
   const int d2 = ghost_step(k, g.N[2]);
   if((d0 | d1 | d2) == 0) return;
 #pragma unroll 1
@@ -637,7 +643,7 @@ __global__ void __launch_bounds__(256) k_fold_copy(Geo g, int nrows, int copy, f
     k0 = layer(tid - r * 2 * HALO, g.N[2]);
     k1 = k0 + 1;
   }
-  const int d0 = ghost_step(i, g.N[0]) * g.L[1] * g.L[2], d1 = ghost_step(j, g.N[1]) * g.L[2];
+  const int d0 = ghost_row(g, i, 0), d1 = ghost_row(g, j, 1);
   for(int k = k0; k < k1; k += int(blockDim.x)) {
     const int d2 = ghost_step(k, g.N[2]);
     if((d0 | d1 | d2) == 0) continue;
