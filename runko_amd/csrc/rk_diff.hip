@@ -148,7 +148,7 @@ struct CurlB {
 };
 
 // The grid of a per-box launch (grid_of, block_of) as part of a launch of 1D
-// workgroups of DWG threads.
+// workgroups of DWG threads (at most MERGED_BLOCKS of them, see merged()).
 struct BoxGrid {
   int gx, gy, gz, bx, by;
   __host__ __device__ int blocks() const { return gx * gy * gz; }
@@ -1627,9 +1627,19 @@ inline BoxGrid box_grid(const DiffImpl& h)
 // Launches are merged where they bound the step: particle blocks of DWG threads
 // with a particle each (up to 2^17 particles) and up to 2^18 cells, beyond which
 // the curls' rows (a workgroup of DWG threads however short) outweigh a launch.
+// The merged launch lays the padded grid of the boxes (the largest side of every
+// axis, times the boxes) out along x.  Boxes of one shape need at most 2^16
+// blocks of it (every block holds two rows of two cells and more); boxes that
+// are long along different axes need up to 2^31 and more, almost all empty, and
+// a grid of 2^24 blocks of DWG threads is past what a launch takes: those keep
+// the launches of their own, whose grid has three dimensions.
+constexpr int64_t MERGED_BLOCKS = int64_t(1) << 16;
+
 inline bool merged(const DiffImpl& h)
 {
-  return h.np > 0 && h.bin_k == 1 && h.bin_threads == DWG && h.ncell <= (int64_t(1) << 18);
+  const dim3 g = grid_of(h);
+  return h.np > 0 && h.bin_k == 1 && h.bin_threads == DWG && h.ncell <= (int64_t(1) << 18) &&
+         int64_t(g.x) * g.y * g.z <= MERGED_BLOCKS;
 }
 
 // the bins of the particles, and before them the curls (c2: if c2.out is given)

@@ -33,12 +33,21 @@ def random_state(box, n, npart, gen, dtype, umax=0.8, famp=0.05):
     return E, B, x, u
 
 
-def build(dtype, seed=3):
+# long along different axes: the grid padded to the longest side of every axis has
+# 1.3e7 workgroups, far more than the boxes' rows
+UNEVEN = [
+    dict(n=(2048, 2, 2), charges=[-0.02, 0.02], masses=[1.0, 1.0], counts=[700, 600]),
+    dict(n=(2, 2048, 2), charges=[-0.01], masses=[1.0], counts=[500]),
+    dict(n=(2, 2, 64), charges=[-0.02, 0.02], masses=[1.0, 1.0], counts=[90, 80]),
+]
+
+
+def build(dtype, seed=3, boxes=BOXES):
     gen = torch.Generator(device="cuda")
     gen.manual_seed(seed)
-    ens = DiffEnsemble(BOXES, cfl=0.45, filter_passes=3, dtype=dtype)
+    ens = DiffEnsemble(boxes, cfl=0.45, filter_passes=3, dtype=dtype)
     singles, states = [], []
-    for bx in BOXES:
+    for bx in boxes:
         b = DiffBox(bx["n"], bx["charges"], bx["masses"], bx["counts"], cfl=0.45, filter_passes=3, dtype=dtype)
         singles.append(b)
         states.append(random_state(b, tuple(bx["n"]), b.np, gen, dtype))
@@ -49,10 +58,14 @@ def build(dtype, seed=3):
     return ens, singles, states, cat
 
 
-@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
-def test_ensemble_step_matches_single_boxes(dtype):
-    ens, singles, states, cat = build(dtype)
-    assert ens.n_boxes == len(BOXES) and ens.np == sum(b.np for b in singles)
+cases = pytest.mark.parametrize("dtype, boxes", [(torch.float32, BOXES), (torch.float64, BOXES), (torch.float64, UNEVEN)],
+                                ids=["fp32", "fp64", "fp64-uneven"])
+
+
+@cases
+def test_ensemble_step_matches_single_boxes(dtype, boxes):
+    ens, singles, states, cat = build(dtype, boxes=boxes)
+    assert ens.n_boxes == len(boxes) and ens.np == sum(b.np for b in singles)
     out = ens.step(cat)
     ftol = 1e-6 if dtype == torch.float32 else 1e-12
     for i, (b, st) in enumerate(zip(singles, states)):
@@ -64,9 +77,9 @@ def test_ensemble_step_matches_single_boxes(dtype):
     assert ens.error_count() == 0
 
 
-@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
-def test_ensemble_adjoint_matches_single_boxes(dtype):
-    ens, singles, states, cat = build(dtype, seed=4)
+@cases
+def test_ensemble_adjoint_matches_single_boxes(dtype, boxes):
+    ens, singles, states, cat = build(dtype, seed=4, boxes=boxes)
     gen = torch.Generator(device="cuda")
     gen.manual_seed(9)
     lam = tuple(torch.randn(t.shape, generator=gen, device="cuda", dtype=torch.float64).to(dtype) for t in cat)
