@@ -978,11 +978,26 @@ __device__ inline int window_node(const BrickOf& bk, const int rel[3], const int
   return in ? (w[0] * D + w[1]) * D + w[2] : -1;
 }
 
-// box node at offsets o of a segment's cell
+// a segment's cell in the box, however far (a large cfl) it lies outside
+struct BoxCell {
+  int c[3];
+};
+
 template<class T>
-__device__ inline int64_t box_node(const DBox<T>& b, const int i[3], const int o[3])
+__device__ inline BoxCell box_cell(const DBox<T>& b, int i0, int i1, int i2)
 {
-  return cidx(b.n, wrap2(i[0] + o[0], b.n[0]), wrap2(i[1] + o[1], b.n[1]), wrap2(i[2] + o[2], b.n[2]));
+  auto rem = [](int i, int n) {
+    const int r = i % n;
+    return r < 0 ? r + n : r;
+  };
+  return BoxCell {{rem(i0, b.n[0]), rem(i1, b.n[1]), rem(i2, b.n[2])}};
+}
+
+// box node at offsets o (0 or 1) of a cell
+template<class T>
+__device__ inline int64_t box_node(const DBox<T>& b, const BoxCell& k, const int o[3])
+{
+  return cidx(b.n, wrap1(k.c[0] + o[0], b.n[0]), wrap1(k.c[1] + o[1], b.n[1]), wrap1(k.c[2] + o[2], b.n[2]));
 }
 
 __device__ inline void lds_add(double* p, double v)
@@ -1068,7 +1083,7 @@ __device__ __attribute__((noinline)) void deposit_far(const DBox<T>& b, T* J0, T
                                                      T F0, T F1, T F2, T W0, T W1, T W2)
 {
   T* const J[3] = {J0, J1, J2};
-  const int i[3] = {i0, i1, i2};
+  const BoxCell k = box_cell(b, i0, i1, i2);
   const T F[3] = {F0, F1, F2}, W[3] = {W0, W1, W2};
   T v[7][3];
   zig_values(F, W, v);
@@ -1076,7 +1091,7 @@ __device__ __attribute__((noinline)) void deposit_far(const DBox<T>& b, T* J0, T
   for(int m = 0; m < 7; ++m)
 #pragma unroll
     for(int c = 0; c < 3; ++c)
-      if(zig_has(m, c)) atomic_add(&J[c][box_node(b, i, ZOFF[m])], v[m][c]);
+      if(zig_has(m, c)) atomic_add(&J[c][box_node(b, k, ZOFF[m])], v[m][c]);
 }
 
 // the forward step of one brick's particles; results go to `out`, which is A
@@ -1278,7 +1293,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(
     } else {
       // a segment further than a cell from the base cell (cfl > 1)
       auto in_box_at = [&](const int* i) {
-        return [&b, &L, i](int d, const int o[3]) { return -L.c[d][box_node(b, i, o)]; };
+        return [&b, &L, k = box_cell(b, i[0], i[1], i[2])](int d, const int o[3]) { return -L.c[d][box_node(b, k, o)]; };
       };
       zig_seg_adj(in_box_at(z.i1), z.F1, z.W1, gF1, gW1);
       zig_seg_adj(in_box_at(z.i2), z.F2, z.W2, gF2, gW2);

@@ -42,7 +42,10 @@ def random_state(n, counts, seed):
     ((264, 256, 256), (60000, 60000), 0.45),  # sorted by groups of 2^3 bricks
 ])
 def test_brick_layouts(n, counts, cfl):
-    s = random_state(n, counts, seed=sum(n))
+    check_step(n, counts, cfl, random_state(n, counts, seed=sum(n)))
+
+
+def check_step(n, counts, cfl, s):
     box = DiffBox(n, Q, M, counts, cfl=cfl, dtype=torch.float64)
     q = tp.per_particle(Q, counts, torch.float64, DEV)
     qm = tp.per_particle([np.sign(a) / b for a, b in zip(Q, M)], counts, torch.float64, DEV)
@@ -57,6 +60,15 @@ def test_brick_layouts(n, counts, cfl):
     for name, a, b in zip("EBxu", box.step_adjoint(s, cot), grad):
         assert rel(a, b) < 1e-9, name
     assert box.error_count() == 0
+
+
+def test_segments_several_boxes_away():
+    # up to 5.5 cells a step along a side of 2: the current's cells lie up to
+    # three sides from the box
+    n, counts = (2, 3, 5), (40, 23)
+    E, B, x, u = random_state(n, counts, seed=11)
+    u[0], u[1:] = 5.0 + u[0].abs(), 0.1 * u[1:]
+    check_step(n, counts, 5.5, (E, B, x, u))
 
 
 def test_particles_outside_the_box_pass_through():
