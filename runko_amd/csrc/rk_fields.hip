@@ -112,7 +112,7 @@ struct StencilM {
 // at(ax, o1, o2) reads the field at offset ax along the derivative's axis a
 // and o1, o2 along the cyclic perpendicular axes (a+1)%3, (a+2)%3
 // AXIAL: rows 1 and 2 have coefficients on the axial line only; their other
-// terms, 0 times a finite difference each, are left out
+// terms, 0 times a finite difference each (stencil_store), are left out
 template<bool AXIAL, class At>
 __device__ inline float stencil_sum(At&& at, const float (&M)[3][5])
 {
@@ -173,10 +173,11 @@ __device__ inline void stencil_load(const Geo& g, float (&v)[SROWS][SLANES], int
   }
 }
 
-// true if a value of this lane is an infinity or a NaN
+// true if a value of this lane is 2^125 or more, an infinity or a NaN: below
+// that the difference of two sums of two values is finite
 __device__ inline bool stencil_store(float (&E)[3][6 * SPL], int slot, const float (&v)[SROWS][SLANES])
 {
-  float zero = 0.0f;
+  uint32_t big = 0;  // bits of the largest magnitude (an infinity's, then a NaN's, are larger)
   const int wave = __builtin_amdgcn_readfirstlane((int(threadIdx.y) * BX + int(threadIdx.x)) / 64);
   const int lane = int(threadIdx.x) % 64;
 #pragma unroll
@@ -186,9 +187,9 @@ __device__ inline bool stencil_store(float (&E)[3][6 * SPL], int slot, const flo
     for(int h = 0; h < SLANES; ++h)
       if(row < 3 * SSY && lane + 64 * h < SSZ) E[c][slot * SPL + y * SSZ + lane + 64 * h] = v[q][h];
 #pragma unroll
-    for(int h = 0; h < SLANES; ++h) zero = zero + v[q][h] * 0.0f;
+    for(int h = 0; h < SLANES; ++h) big = max(big, __float_as_uint(fabsf(v[q][h])));
   }
-  return !(zero == 0.0f);
+  return big >= __float_as_uint(0x1p125f);
 }
 
 // derivative along axis A of the staged component Ec at the ring cell `cell`;
@@ -211,7 +212,7 @@ __device__ inline float stencil_lds(const float* Ec, const int (&sb)[6], int cel
 // segments are too few blocks, latency.  `axial` (the coefficients of the
 // reference's shock configuration, projects/pic-shock/3d_shock.ini:48-70, are of
 // that form) takes 132 reads as long as every value that the block has staged
-// is finite.  512 x 64 x 64 cells: 130 us in segments of 32 planes (256 blocks),
+// is below 2^125.  512 x 64 x 64 cells: 130 us in segments of 32 planes (256 blocks),
 // 89 us in segments of 8, 63 us axial.
 __global__ void __launch_bounds__(BX* BY)
   k_curl_b_stencil(Geo g, Region r, float dt, StencilM S, int xseg, int axial, const float* __restrict__ Ex,
