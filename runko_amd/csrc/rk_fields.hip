@@ -14,6 +14,7 @@
 // contiguous dimension), 4 rows along y per workgroup, one x plane per
 // grid.z, so every wave reads 256 contiguous bytes per component.
 #include "rk_internal.h"
+#include "rk_ghost.h"
 
 #include <cmath>
 #include <cstring>
@@ -38,7 +39,7 @@ inline dim3 region_grid(const Region& r)
 }
 
 // A periodic world with at least 2 * HALO cells along every axis: an interior
-// node has at most one image in the ghost shell along an axis, ghost_step away.
+// node has at most one image in the ghost shell along an axis (rk_ghost.h).
 // A kernel that computes whole fields stores a node's new value into its (up to
 // 7) images as well (`ghosts`), so no launch has to copy the ghost shell after
 // it: at 64^3 such a copy takes 5 us, as long as the kernel before it.
@@ -47,24 +48,17 @@ bool ghosts_in_pass(const Geo& g)
   return g.periodic && g.N[0] >= 2 * HALO && g.N[1] >= 2 * HALO && g.N[2] >= 2 * HALO;
 }
 
-__device__ inline int ghost_step(int c, int N) { return c < 2 * HALO ? N : (c >= N ? -N : 0); }
-// the step along axis 0 or 1 as an offset in the lattice (modulo 2^32, as its indices)
-__device__ inline int ghost_row(const Geo& g, int c, int axis)
-{
-  const uint32_t row = axis == 0 ? uint32_t(g.L[1]) * uint32_t(g.L[2]) : uint32_t(g.L[2]);
-  return int(uint32_t(ghost_step(c, g.N[axis])) * row);
-}
+static_assert(GHOST_LAYERS == HALO, "one halo width");
 
 __device__ inline void put_ghosts(const Geo& g, int i, int j, int k, uint32_t c, float* F0, float* F1, float* F2,
                                   float v0, float v1, float v2)
 {
-  const int d0 = ghost_row(g, i, 0), d1 = ghost_row(g, j, 1);
-  const int d2 = ghost_step(k, g.N[2]);
+  const uint32_t d0 = ghost_row(g.N, g.L, i, 0), d1 = ghost_row(g.N, g.L, j, 1), d2 = ghost_step(k, g.N[2]);
   if((d0 | d1 | d2) == 0) return;
 #pragma unroll 1
   for(int n = 1; n < 8; ++n) {
-    if(((n & 4) && !d0) || ((n & 2) && !d1) || ((n & 1) && !d2)) continue;
-    const uint32_t q = c + uint32_t((n & 4 ? d0 : 0) + (n & 2 ? d1 : 0) + (n & 1 ? d2 : 0));
+    if(!ghost_there(n, d0, d1, d2)) continue;
+    const uint32_t q = c + ghost_image(n, d0, d1, d2);
     F0[q] = v0;
     F1[q] = v1;
     F2[q] = v2;
@@ -644,31 +638,30 @@ __global__ void __launch_bounds__(256) k_fold_copy(Geo g, int nrows, int copy, f
     k0 = layer(tid - r * 2 * HALO, g.N[2]);
     k1 = k0 + 1;
   }
-  const int d0 = ghost_row(g, i, 0), d1 = ghost_row(g, j, 1);
+  const uint32_t d0 = ghost_row(g.N, g.L, i, 0), d1 = ghost_row(g.N, g.L, j, 1);
   for(int k = k0; k < k1; k += int(blockDim.x)) {
-    const int d2 = ghost_step(k, g.N[2]);
+    const uint32_t d2 = ghost_step(k, g.N[2]);
     if((d0 | d1 | d2) == 0) continue;
     const uint32_t c = g.at(i, j, k);
     uint32_t q[8];
     float v[8];
 #pragma unroll
     for(int n = 0; n < 8; ++n) {
-      q[n] = c + uint32_t((n & 4 ? d0 : 0) + (n & 2 ? d1 : 0) + (n & 1 ? d2 : 0));
+      q[n] = c + ghost_image(n, d0, d1, d2);
       v[n] = F[q[n]];  // an image that is not there reads another of the eight
     }
-    auto there = [&](int n) { return (!(n & 4) || d0 != 0) && (!(n & 2) || d1 != 0) && (!(n & 1) || d2 != 0); };
     float sum = v[0];
 #pragma unroll
     for(int n = 1; n < 8; ++n) {
       asm volatile("" : "+v"(v[n]));  // keeps the loads together, ahead of the conditions
       const float t = sum + v[n];
-      sum = there(n) ? t : sum;
+      sum = ghost_there(n, d0, d1, d2) ? t : sum;
     }
     F[c] = sum;
     if(copy) {
 #pragma unroll
       for(int n = 1; n < 8; ++n)
-        if(there(n)) F[q[n]] = sum;
+        if(ghost_there(n, d0, d1, d2)) F[q[n]] = sum;
     }
   }
 }
