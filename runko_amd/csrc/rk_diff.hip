@@ -661,7 +661,8 @@ __device__ inline int species_of(const DBox<T>& b, int64_t p)
 //              there in double precision; each record's result replaces it;
 //   k_dunsort  a block puts its P records back in the arrays' order.
 // The sort never leaves a block, so records move only inside P slots that
-// stay in cache, with no global atomic and no scan over bricks.  About 220
+// stay in cache, with no global atomic and no scan over bricks (boxes of more
+// than GROUPS_MAX bricks need both, see k_dcount).  About 220
 // bytes per particle and step cross memory; the pass over 96^3 cells with 2.8e7
 // mixed particles takes 2.3 ms (7.3 ms with random corner reads, records
 // bucketed by cell through global counters and a scan), its adjoint 3.8 ms
@@ -792,8 +793,6 @@ bin_block(int block, const DEnt<T>* __restrict__ tab, const uint16_t* __restrict
         for(int a = 0; a < 6; ++a) r.v[a] = lr[k][a];
         r.v[6] = T(0);
         B[at] = r;
-      } else if(key == en.ngroup) {
-        B[at] = r;  // outside the box: the step passes it through
       }
     }
   }
@@ -844,6 +843,146 @@ __global__ void __launch_bounds__(1024)
   unsort_block<T, K>(int(blockIdx.x), tab, pmap, slot, A, x, u);
 }
 
+// Boxes of more than GROUPS_MAX bricks, whose rows hold runs of groups of bricks:
+// a brick's records through a list of their places, sorted by brick.  A record
+// takes its number in its brick from a global counter (k_dcount), the counters
+// become the bricks' starts (k_dsums, k_dstarts), and the places are stored
+// (k_dorder).  A brick that walked its group's runs passed over the other
+// bricks' records with most lanes idle: 512^3 cells, groups of 4^3, 1.34e8 mixed
+// particles took 145 ms a step and 279 ms its adjoint, 31 and 46 ms so; 256^3
+// cells, groups of 2^3, 27 and 50 ms, 18 and 25.5 so (k_dcount 2.4, k_dorder 2.3
+// ms of each, bound by their scattered 4-byte accesses).
+template<class T>
+__device__ inline int64_t brick_number(const DEnt<T>& en, const T x[3])
+{
+  int k[3];
+#pragma unroll
+  for(int a = 0; a < 3; ++a) {
+    T d;
+    k[a] = brick_at(en.ax[a], wrap2(base_cell(x[a], d), en.b.n[a]));
+  }
+  return en.k0 + (int64_t(k[0]) * en.ax[1].nb + k[1]) * en.ax[2].nb + k[2];
+}
+
+// a lane's number among those that take one of counter `key`: an atomic for all
+// lanes of one key while they are many (particles in cell order), else one each
+__device__ inline uint32_t take_number(uint32_t* __restrict__ count, int64_t key, bool live)
+{
+  const int lane = int(threadIdx.x) & 63;
+  const uint64_t below = (uint64_t(1) << lane) - 1;
+  uint64_t left = __ballot(live);
+  while(left) {
+    const int lead = __ffsll(static_cast<unsigned long long>(left)) - 1;
+    const int64_t k = __shfl(key, lead);
+    const uint64_t same = __ballot(live && key == k) & left;
+    if(__popcll(same) < 8) break;
+    uint32_t base = 0;
+    if(lane == lead) base = atomicAdd(&count[k], uint32_t(__popcll(same)));
+    base = __shfl(base, lead);
+    if(same >> lane & 1) return base + uint32_t(__popcll(same & below));
+    left &= ~same;
+  }
+  return (left >> lane & 1) ? atomicAdd(&count[key], 1u) : 0u;
+}
+
+constexpr uint32_t NO_RANK = UINT32_MAX;
+
+template<class T>
+__global__ void __launch_bounds__(DWG)
+  k_dcount(const DEnt<T>* __restrict__ tab, const uint16_t* __restrict__ pmap, int64_t P, const Rec<T>* __restrict__ A,
+           uint32_t* __restrict__ count, uint32_t* __restrict__ rank)
+{
+  const DEnt<T>& en = tab[pmap[blockIdx.x]];
+  const int64_t p0 = (int64_t(blockIdx.x) - en.pb0) * P, p1 = min(p0 + P, en.b.off[en.b.nsp]);
+  for(int64_t q0 = p0; q0 < p1; q0 += DWG) {
+    const int64_t q = q0 + threadIdx.x, at = en.p0 + min(q, p1 - 1);
+    const T x[3] = {A[at].v[0], A[at].v[1], A[at].v[2]};
+    const bool live = q < p1 && in_box(en.b, x);
+    const uint32_t r = take_number(count, live ? brick_number(en, x) : 0, live);
+    if(q < p1) rank[at] = live ? r : NO_RANK;
+  }
+}
+
+constexpr int SCAN = 4096;  // counters of a workgroup
+
+__device__ inline uint32_t block_sum(uint32_t v, uint32_t* wsum)
+{
+#pragma unroll
+  for(int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  __syncthreads();
+  if((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = v;
+  __syncthreads();
+  uint32_t sum = 0;
+#pragma unroll
+  for(int w = 0; w < DWG / 64; ++w) sum += wsum[w];
+  return sum;
+}
+
+static __global__ void __launch_bounds__(DWG) k_dzero(uint32_t* __restrict__ p, int64_t n)
+{
+  const int64_t i = int64_t(blockIdx.x) * DWG + threadIdx.x;
+  if(i < n) p[i] = 0;
+}
+
+static __global__ void __launch_bounds__(DWG) k_dsums(const uint32_t* __restrict__ count, int64_t n, uint32_t* __restrict__ sums)
+{
+  __shared__ uint32_t wsum[DWG / 64];
+  const int64_t c0 = int64_t(blockIdx.x) * SCAN, c1 = min(c0 + SCAN, n);
+  uint32_t v = 0;
+  for(int64_t c = c0 + threadIdx.x; c < c1; c += DWG) v += count[c];
+  v = block_sum(v, wsum);
+  if(threadIdx.x == 0) sums[blockIdx.x] = v;
+}
+
+// counts -> exclusive starts, in place; entry n takes the total
+static __global__ void __launch_bounds__(DWG)
+  k_dstarts(uint32_t* __restrict__ count, int64_t n, const uint32_t* __restrict__ sums)
+{
+  __shared__ uint32_t wsum[DWG / 64];
+  uint32_t v = 0;
+  for(int b = int(threadIdx.x); b < int(blockIdx.x); b += DWG) v += sums[b];
+  uint32_t run = block_sum(v, wsum);
+  const int64_t c0 = int64_t(blockIdx.x) * SCAN, c1 = min(c0 + SCAN, n);
+  const int wave = int(threadIdx.x) >> 6;
+  for(int64_t q = c0; q < c1; q += DWG) {
+    const int64_t c = q + threadIdx.x;
+    const uint32_t own = c < c1 ? count[c] : 0;
+    uint32_t inc = own;
+#pragma unroll
+    for(int o = 1; o < 64; o <<= 1) {
+      const uint32_t t = __shfl_up(inc, o);
+      if((int(threadIdx.x) & 63) >= o) inc += t;
+    }
+    __syncthreads();
+    if((threadIdx.x & 63) == 63) wsum[wave] = inc;
+    __syncthreads();
+    uint32_t before = run;
+#pragma unroll
+    for(int w = 0; w < DWG / 64; ++w) {
+      before += w < wave ? wsum[w] : 0;
+      run += wsum[w];
+    }
+    if(c < c1) count[c] = before + inc - own;
+  }
+  if(c1 == n && threadIdx.x == 0) count[n] = run;
+}
+
+template<class T>
+__global__ void __launch_bounds__(DWG)
+  k_dorder(const DEnt<T>* __restrict__ tab, const uint16_t* __restrict__ pmap, int64_t P, const Rec<T>* __restrict__ A,
+           const uint32_t* __restrict__ start, const uint32_t* __restrict__ rank, uint32_t* __restrict__ order)
+{
+  const DEnt<T>& en = tab[pmap[blockIdx.x]];
+  const int64_t p0 = (int64_t(blockIdx.x) - en.pb0) * P, p1 = min(p0 + P, en.b.off[en.b.nsp]);
+  for(int64_t q = p0 + threadIdx.x; q < p1; q += DWG) {
+    const int64_t at = en.p0 + q;
+    const uint32_t r = rank[at];
+    if(r == NO_RANK) continue;
+    const T x[3] = {A[at].v[0], A[at].v[1], A[at].v[2]};
+    order[start[brick_number(en, x)] + r] = uint32_t(at);
+  }
+}
+
 // Small boxes (a particle a thread in the particle blocks): a launch costs
 // about 4 us whatever it does, so what needs nothing of each other shares one.
 // Before the bricks' step, the particles' bins and the curls of the fields; a
@@ -889,7 +1028,6 @@ __global__ void __launch_bounds__(DWG)
 // one brick of a box
 struct BrickOf {
   int s[3], n[3];  // first cell, cells
-  int group;       // its run in every row
 };
 
 template<class T>
@@ -898,14 +1036,11 @@ __device__ inline BrickOf brick_of_box(const DEnt<T>& en, int64_t k)
   BrickOf B;
   const uint32_t kk = uint32_t(k), n1 = uint32_t(en.ax[1].nb), n2 = uint32_t(en.ax[2].nb);
   const int kc[3] = {int(kk / n2 / n1), int(kk / n2 % n1), int(kk % n2)};
-  int g[3];
 #pragma unroll
   for(int a = 0; a < 3; ++a) {
     B.s[a] = brick_start(en.ax[a], kc[a]);
     B.n[a] = brick_start(en.ax[a], kc[a] + 1) - B.s[a];
-    g[a] = kc[a] >> en.gsh;
   }
-  B.group = (g[0] * en.ng[1] + g[1]) * en.ng[2] + g[2];
   return B;
 }
 
@@ -1005,20 +1140,47 @@ __device__ inline void lds_add(double* p, double v)
   __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// The records of one brick, taken by its workgroup's NT threads: rows are
+// Where a brick's records are: its run in the row of every particle block, or,
+// in a box of more than GROUPS_MAX bricks, its part of a list (k_dorder).
+struct Runs {
+  const uint32_t* rows;
+  int64_t P;
+  const uint32_t *bstart, *order;
+};
+
+// The records of brick k of a box, taken by its workgroup's NT threads: rows are
 // scanned NT at a time; a thread takes a contiguous share of the records they
 // hold, so neighbouring lanes are far apart in a run (the particles of a cell
 // that lie one after the other go to one lane, and the lanes' LDS adds to
-// different nodes).  body(first record of the row's block, slot).
-template<class T, int NT, class Body>
-__device__ inline void for_records(const DEnt<T>& en, const uint32_t* __restrict__ rows, int group, int64_t P,
-                                   const Rec<T>* A, Body&& body)
+// different nodes).  body(record, its place).
+template<class T, int NT, bool LIST, class Body>
+__device__ inline void for_records(const DEnt<T>& en, const Runs& runs, int64_t k, const Rec<T>* A, Body&& body)
 {
+  const int tid = int(threadIdx.x);
+  if constexpr(LIST) {
+    const uint32_t lo = runs.bstart[en.k0 + k], total = runs.bstart[en.k0 + k + 1] - lo;
+    const uint32_t* __restrict__ const list = runs.order + lo;
+    const uint32_t per = (total + NT - 1) / NT, end = min((uint32_t(tid) + 1) * per, total);
+    uint32_t r = min(uint32_t(tid) * per, total);
+    if(r >= end) return;
+    int64_t at = list[r];
+    Rec<T> rec = A[at];
+    for(; r < end; ++r) {
+      const int64_t here = at;
+      const Rec<T> cur = rec;
+      if(r + 1 < end) {
+        at = list[r + 1];
+        rec = A[at];
+      }
+      body(cur, here);
+    }
+    return;
+  }
   __shared__ uint32_t pre[NT + 1];  // records of the rows before
   __shared__ uint16_t first[NT];
   __shared__ uint32_t wsum[NT / 64];
-  const int tid = int(threadIdx.x);
-  const uint16_t* tabl = reinterpret_cast<const uint16_t*>(rows + en.row0) + group;
+  const int64_t P = runs.P;
+  const uint16_t* tabl = reinterpret_cast<const uint16_t*>(runs.rows + en.row0) + k;
   const int64_t stride = 2 * int64_t(en.rowlen);
   for(int64_t r0 = 0; r0 < en.nrow; r0 += NT) {
     uint32_t a = 0, len = 0;
@@ -1094,37 +1256,35 @@ __device__ __attribute__((noinline)) void deposit_far(const DBox<T>& b, T* J0, T
       if(zig_has(m, c)) atomic_add(&J[c][box_node(b, k, ZOFF[m])], v[m][c]);
 }
 
-// the forward step of one brick's particles; results go to `out`, which is A
-// itself (a second set of records made the step 12 to 35 % slower: twice the
-// lines to hold in cache) unless other bricks read the same run
-template<class T, int BR, int NT>
+// the forward step of one brick's particles; results replace the records (a
+// second set of records made the step 12 to 35 % slower: twice the lines to
+// hold in cache)
+template<class T, int BR, int NT, bool LIST>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 5 : 4)))
   k_dstep(const DEnt<T>* __restrict__ tab, const uint16_t* __restrict__ kmap, G3<T> E, G3<T> B,
-          const uint32_t* __restrict__ rows, int64_t P, const Rec<T>* A, Rec<T>* out, T* __restrict__ jst, G3<T> J)
+          Runs runs, Rec<T>* A, T* __restrict__ jst, G3<T> J)
 {
   constexpr int M = BR + 1, D = BR + 3, V = D * D * D;
   __shared__ double win[3 * V];
   __shared__ T nm[6 * M * M * M];
   const DEnt<T>& en = tab[kmap[blockIdx.x]];
   const DBox<T>& b = en.b;
-  const BrickOf bk = brick_of_box(en, int64_t(blockIdx.x) - en.k0);
+  const int64_t kb = int64_t(blockIdx.x) - en.k0;
+  const BrickOf bk = brick_of_box(en, kb);
   E = sh(E, en.c0);
   B = sh(B, en.c0);
   J = sh(J, en.c0);
   for(int q = int(threadIdx.x); q < 3 * V; q += NT) win[q] = 0.0;
   stage_nodes<T, BR, NT>(b, bk, E, B, nm);
   __syncthreads();
-  for_records<T, NT>(en, rows, bk.group, P, A, [&](Rec<T> r, int64_t at) {
+  for_records<T, NT, LIST>(en, runs, kb, A, [&](Rec<T> r, int64_t at) {
     Fwd<T> f;
     int cell[3], l[3];
-    bool mine = true;
 #pragma unroll
     for(int a = 0; a < 3; ++a) {
       cell[a] = base_cell(r.v[a], f.d[a]);
       l[a] = wrap2(cell[a], b.n[a]) - bk.s[a];
-      mine = mine && l[a] >= 0 && l[a] < bk.n[a];
     }
-    if(!mine) return;  // another brick of the group
     const int s = int(r.v[6]);
     gather_nodes<T, BR>(nm, (l[0] * M + l[1]) * M + l[2], f);
     BorisT<T> bs;
@@ -1137,7 +1297,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(
       r.v[a] = f.xw[a];
       r.v[3 + a] = f.un[a];
     }
-    out[at] = r;
+    A[at] = r;
     int rel[3];
     window_rel(b, l, cell, f.xn, rel);
     const int o1 = window_node<BR>(bk, rel, z.i1), o2 = window_node<BR>(bk, rel, z.i2);
@@ -1225,11 +1385,10 @@ __device__ inline void cross_adj(const T a[3], const T b[3], const T gc[3], T ga
 // at the particle times the trilinear weights of its 8 corners) to the
 // brick's window; records of A (x, u) stay, records of B (lambda_x, lambda_u)
 // are replaced.
-template<class T, int BR, int NT>
+template<class T, int BR, int NT, bool LIST>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 2)))
   k_dadj(const DEnt<T>* __restrict__ tab, const uint16_t* __restrict__ kmap, G3<T> E, G3<T> B, G3<T> L,
-         const uint32_t* __restrict__ rows, int64_t P, const Rec<T>* __restrict__ A, Rec<T>* __restrict__ lam,
-         T* __restrict__ mst)
+         Runs runs, const Rec<T>* __restrict__ A, Rec<T>* __restrict__ lam, T* __restrict__ mst)
 {
   constexpr int M = BR + 1, MV = M * M * M, D = BR + 3, V = D * D * D;
   __shared__ double mw[6 * MV];
@@ -1237,7 +1396,8 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(
   __shared__ T lw[3 * V];
   const DEnt<T>& en = tab[kmap[blockIdx.x]];
   const DBox<T>& b = en.b;
-  const BrickOf bk = brick_of_box(en, int64_t(blockIdx.x) - en.k0);
+  const int64_t kb = int64_t(blockIdx.x) - en.k0;
+  const BrickOf bk = brick_of_box(en, kb);
   E = sh(E, en.c0);
   B = sh(B, en.c0);
   L = sh(L, en.c0);
@@ -1255,18 +1415,15 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(
   }
   __syncthreads();
   const T cfl = b.cfl;
-  for_records<T, NT>(en, rows, bk.group, P, A, [&](const Rec<T>& r, int64_t at) {
+  for_records<T, NT, LIST>(en, runs, kb, A, [&](const Rec<T>& r, int64_t at) {
     Rec<T> g = lam[at];
     Fwd<T> f;
     int cell[3], l[3];
-    bool mine = true;
 #pragma unroll
     for(int a = 0; a < 3; ++a) {
       cell[a] = base_cell(r.v[a], f.d[a]);
       l[a] = wrap2(cell[a], b.n[a]) - bk.s[a];
-      mine = mine && l[a] >= 0 && l[a] < bk.n[a];
     }
-    if(!mine) return;  // another brick of the group
     const int s = int(r.v[6]);
     const int node = (l[0] * M + l[1]) * M + l[2];
     const T gxo[3] = {g.v[0], g.v[1], g.v[2]}, guo[3] = {g.v[3], g.v[4], g.v[5]};
@@ -1433,13 +1590,17 @@ struct DiffImpl {
   int bin_threads = 256, bin_k = 1;  // a particle block: threads and particles per thread
   int64_t pblocks = 0, nbricks = 0, row_words = 0;
   int rowlen_max = 0;
-  int grouped = 0;                   // 1: some box sorts by groups of bricks
+  bool listed = false;               // some box has too many bricks for a row: records through a list
   uint16_t* pmap = nullptr;          // particle block -> box
   uint16_t* kmap = nullptr;          // brick -> box
   void* scratch[5][3] = {};          // B1, J, Jt, LB2, LE (planar)
-  void* recs[2] = {};                // the sorted blocks' records: x, u; lambda_x, lambda_u (or a grouped step's results)
+  void* recs[2] = {};                // the sorted blocks' records: x, u; lambda_x, lambda_u
   uint16_t* slot = nullptr;          // particle -> its record's slot in its block
   uint32_t* rows = nullptr;          // run starts of every block
+  uint32_t* rank = nullptr;          // listed: a record's number in its brick
+  uint32_t* order = nullptr;         // listed: the records' places, sorted by brick
+  uint32_t* bstart = nullptr;        // listed: the bricks' starts in it
+  uint32_t* bsums = nullptr;         // listed: sums of SCAN counters each
   void* stage = nullptr;             // per brick: its current or node-mean adjoint window
   unsigned long long* err = nullptr;
 };
@@ -1485,7 +1646,9 @@ constexpr int GROUPS_MAX = 32000;
 //    piece.  2.8e7 mixed particles, P = 4096 and 8192: k_dbin<adjoint> + k_dadj
 //    3.43 and 3.33 ms; 4.2e6 particles in cell order: k_dbin 60 and 66 us.
 //  * Boxes of more than GROUPS_MAX bricks sort by groups of 2^gsh bricks per
-//    axis; a brick then passes over its group's other records.
+//    axis, and their bricks take the records through a list (k_dorder).  Just
+//    below and above the line, 1.34e8 mixed particles: 248 x 256 x 256 cells 16.6
+//    ms a step and 30 ms its adjoint, 256^3 17.9 and 25.5 ms.
 template<class T>
 hipError_t upload_table(DiffImpl& h)
 {
@@ -1521,7 +1684,7 @@ hipError_t upload_table(DiffImpl& h)
     h.pblocks += e.nrow;
     h.row_words += e.nrow * e.rowlen;
     h.rowlen_max = std::max(h.rowlen_max, e.rowlen);
-    if(e.gsh > 0) h.grouped = 1;
+    if(e.gsh > 0) h.listed = true;
     pm.resize(size_t(h.pblocks), uint16_t(i));
     km.resize(size_t(h.nbricks), uint16_t(i));
   }
@@ -1541,6 +1704,13 @@ hipError_t upload_table(DiffImpl& h)
   if(e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&h.slot), sizeof(uint16_t) * n1);
   if(e == hipSuccess)
     e = hipMalloc(reinterpret_cast<void**>(&h.rows), sizeof(uint32_t) * size_t(std::max<int64_t>(h.row_words, 1)));
+  auto words = [&](uint32_t** p, size_t n) {
+    if(h.listed && e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(p), sizeof(uint32_t) * n);
+  };
+  words(&h.rank, n1);
+  words(&h.order, n1);
+  words(&h.bstart, size_t(h.nbricks) + 1);
+  words(&h.bsums, size_t(h.nbricks + SCAN - 1) / SCAN);
   return e;
 }
 
@@ -1620,6 +1790,30 @@ int bin_particles(const DiffImpl& h, G3<T> x, G3<T> u, G3<T> lx, G3<T> lu, hipSt
   return RK_OK;
 }
 
+// the bricks' lists of their records, where they need them
+template<class T>
+int list_records(const DiffImpl& h, hipStream_t st)
+{
+  if(!h.listed) return RK_OK;
+  const int64_t P = int64_t(h.bin_threads) * h.bin_k;
+  const Rec<T>* A = static_cast<const Rec<T>*>(h.recs[0]);
+  const unsigned scan = unsigned((h.nbricks + SCAN - 1) / SCAN);
+  hipLaunchKernelGGL(k_dzero, dim3(unsigned((h.nbricks + DWG - 1) / DWG)), dim3(DWG), 0, st, h.bstart, h.nbricks);
+  RK_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_dcount<T>, dim3(unsigned(h.pblocks)), dim3(DWG), 0, st, table<T>(h), h.pmap, P, A, h.bstart, h.rank);
+  RK_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_dsums, dim3(scan), dim3(DWG), 0, st, h.bstart, h.nbricks, h.bsums);
+  RK_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_dstarts, dim3(scan), dim3(DWG), 0, st, h.bstart, h.nbricks, h.bsums);
+  RK_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_dorder<T>, dim3(unsigned(h.pblocks)), dim3(DWG), 0, st, table<T>(h), h.pmap, P, A, h.bstart, h.rank,
+                     h.order);
+  RK_HIP(hipGetLastError());
+  return RK_OK;
+}
+
+Runs runs_of(const DiffImpl& h) { return Runs {h.rows, int64_t(h.bin_threads) * h.bin_k, h.bstart, h.order}; }
+
 // the records of set `which` back into x, u in the arrays' order
 template<class T>
 int unsort_particles(const DiffImpl& h, int which, G3<T> x, G3<T> u, hipStream_t st)
@@ -1676,7 +1870,9 @@ int prepare(const DiffImpl& h, G3<T> x, G3<T> u, G3<T> lx, G3<T> lu, const CurlB
     hipLaunchKernelGGL(k_dcurl_b<T>, grid_of(h), block_of(h), 0, st, table<T>(h), c2);
     RK_HIP(hipGetLastError());
   }
-  return h.np > 0 ? bin_particles<T, ADJ>(h, x, u, lx, lu, st) : RK_OK;
+  if(h.np == 0) return RK_OK;
+  if(int rc = bin_particles<T, ADJ>(h, x, u, lx, lu, st)) return rc;
+  return list_records<T>(h, st);
 }
 
 template<class T, int BR>
@@ -1686,26 +1882,28 @@ int step_t(DiffImpl& h, const rk_diff_state* in, rk_diff_state* out, hipStream_t
   const T half = static_cast<T>(h.d.cfl / 2), full = static_cast<T>(h.d.cfl);
   const G3<T> none {{nullptr, nullptr, nullptr}};
   const G3<T> E = g3<T>(in->E), B = g3<T>(in->B), B1 = g3s<T>(h, S_B1), J = g3s<T>(h, S_J);
-  const int64_t P = int64_t(h.bin_threads) * h.bin_k;
   // B1 = B + cfl/2 curlE(E); J = 0
   if(int rc = prepare<T, false>(h, g3<T>(in->x), g3<T>(in->u), none, none, {B1, B, E, half, J}, {none, none, none, half, none}, st))
     return rc;
   if(h.np > 0) {
     constexpr int NT = brick_threads(BR);
     T* jst = static_cast<T*>(h.stage);
-    hipLaunchKernelGGL((k_dstep<T, BR, NT>), dim3(unsigned(h.nbricks)), dim3(NT), 0, st, b, h.kmap, E, B1, h.rows, P,
-                       static_cast<const Rec<T>*>(h.recs[0]), static_cast<Rec<T>*>(h.recs[h.grouped]), jst, J);
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(unsigned(h.nbricks)), dim3(NT), 0, st, b, h.kmap, E, B1, runs_of(h),
+                         static_cast<Rec<T>*>(h.recs[0]), jst, J);
+    };
+    h.listed ? go(k_dstep<T, BR, NT, BR == 8>) : go(k_dstep<T, BR, NT, false>);  // (listed boxes have bricks of 8 cells)
     RK_HIP(hipGetLastError());
     if(merged(h)) {
       const BoxGrid bg = box_grid(h);
       hipLaunchKernelGGL((k_dfinish<T, BR, false>), dim3(unsigned(h.pblocks + bg.blocks())), dim3(DWG), 0, st, b, h.pmap,
-                         h.slot, static_cast<const Rec<T>*>(h.recs[h.grouped]), g3<T>(out->x), g3<T>(out->u),
+                         h.slot, static_cast<const Rec<T>*>(h.recs[0]), g3<T>(out->x), g3<T>(out->u),
                          int(h.pblocks), bg, J, none, none, jst);
       RK_HIP(hipGetLastError());
     } else {
       hipLaunchKernelGGL((k_djgather<T, BR>), grid_of(h), block_of(h), 0, st, b, J, jst);
       RK_HIP(hipGetLastError());
-      if(int rc = unsort_particles<T>(h, h.grouped, g3<T>(out->x), g3<T>(out->u), st)) return rc;
+      if(int rc = unsort_particles<T>(h, 0, g3<T>(out->x), g3<T>(out->u), st)) return rc;
     }
   }
   G3<T> jf = J;
@@ -1727,7 +1925,6 @@ int adjoint_t(DiffImpl& h, const rk_diff_state* in, const rk_diff_state* ao, rk_
   const G3<T> none {{nullptr, nullptr, nullptr}};
   const G3<T> E = g3<T>(in->E), B = g3<T>(in->B), B1 = g3s<T>(h, S_B1);
   const G3<T> LEo = g3<T>(ao->E), LBo = g3<T>(ao->B), LB2 = g3s<T>(h, S_LB2), LE = g3s<T>(h, S_LE);
-  const int64_t P = int64_t(h.bin_threads) * h.bin_k;
   // forward B1, and
   // E' = E + cfl curlB(B2) - Jf:  lambda_B2 = LB' + cfl curlB^T(LE') = LB' - cfl curlE(LE')
   if(int rc = prepare<T, true>(h, g3<T>(in->x), g3<T>(in->u), g3<T>(ao->x), g3<T>(ao->u), {B1, B, E, half, none},
@@ -1743,8 +1940,11 @@ int adjoint_t(DiffImpl& h, const rk_diff_state* in, const rk_diff_state* ao, rk_
     if(int rc = filter_passes<T>(h, b, lj, st)) return rc;
     constexpr int NT = brick_threads(BR);
     T* mst = static_cast<T*>(h.stage);
-    hipLaunchKernelGGL((k_dadj<T, BR, NT>), dim3(unsigned(h.nbricks)), dim3(NT), 0, st, b, h.kmap, E, B1, lj, h.rows, P,
-                       static_cast<const Rec<T>*>(h.recs[0]), static_cast<Rec<T>*>(h.recs[1]), mst);
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(unsigned(h.nbricks)), dim3(NT), 0, st, b, h.kmap, E, B1, lj, runs_of(h),
+                         static_cast<const Rec<T>*>(h.recs[0]), static_cast<Rec<T>*>(h.recs[1]), mst);
+    };
+    h.listed ? go(k_dadj<T, BR, NT, BR == 8>) : go(k_dadj<T, BR, NT, false>);
     RK_HIP(hipGetLastError());
     // node-mean adjoints: lambda_E += NM_E^T(ME), lambda_B = lambda_B1 = LB2 + NM_B^T(MB)
     LB1 = g3<T>(ai->B);
@@ -1854,8 +2054,10 @@ int rk_diff_destroy(rk_diff* h)
   for(auto& s : h->scratch)
     for(auto& p : s)
       if(p) (void)hipFree(p);
-  for(void* q : {h->recs[0], h->recs[1], static_cast<void*>(h->slot), static_cast<void*>(h->rows), h->stage,
-                 static_cast<void*>(h->err), h->tab, static_cast<void*>(h->pmap), static_cast<void*>(h->kmap)})
+  for(void* q : {h->recs[0], h->recs[1], static_cast<void*>(h->slot), static_cast<void*>(h->rows),
+                 static_cast<void*>(h->rank), static_cast<void*>(h->order), static_cast<void*>(h->bstart),
+                 static_cast<void*>(h->bsums), h->stage, static_cast<void*>(h->err), h->tab, static_cast<void*>(h->pmap),
+                 static_cast<void*>(h->kmap)})
     if(q) (void)hipFree(q);
   delete h;
   return RK_OK;
