@@ -250,8 +250,9 @@ int rk_exchange_current(rk_world* w, void* stream);
 /* Kernel timing: when enabled, every launch is bracketed by HIP events on its
  * stream, accumulated per category; rk_profile_read (synchronous) returns and
  * clears the totals.  Categories: 0 fused particle step kernel, 1 push,
- * 2 deposit, 3 pack, 4 migration append (after the fused step with the gather
- * of its current windows, one launch), 5 fdtd curl (+E -= J), 6 filter,
+ * 2 deposit (after the fused step the gather of its current windows, for which
+ * timing takes a launch of its own), 3 pack, 4 migration append, 5 fdtd curl
+ * (+E -= J; in the batched pairs with the ghost images it writes), 6 filter,
  * 7 ghost copy/fold, 8 other (fills, counters, sort).  Not for use while a
  * stream is being captured into a graph. */
 #define RK_PROF_NCAT 9

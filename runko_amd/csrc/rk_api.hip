@@ -695,11 +695,14 @@ int fused_step(rk_world* w, const rk_reflector_wall* walls, int32_t n_walls, boo
     ProfScope ps(w, 0, s);
     if(int rc = launch_fused(w, s, &ws, device_walls ? w->walls_dev : nullptr)) return rc;
   }
+  const bool timed = w->prof_on;
   {
     ProfScope ps(w, 4, s);
-    if(int rc = launch_fused_tail(w, s)) return rc;
+    if(int rc = launch_fused_tail(w, true, !timed, s)) return rc;
   }
   ProfScope ps(w, 2, s);
+  if(timed)
+    if(int rc = launch_fused_tail(w, false, true, s)) return rc;
   if(int rc = apply_corrections(w, -1, s)) return rc;
   return device_walls && ws.n > 0 ? add_corrections_world(w, s) : RK_OK;
 }

@@ -244,8 +244,8 @@ int launch_deposit(rk_world* w, int tile, hipStream_t s);
 int launch_pack(rk_world* w, int tile, hipStream_t s);
 int launch_append(rk_world* w, int set, hipStream_t s);
 // after the fused step: mailboxes and record sets appended (the sets' counters
-// cleared), staged current windows gathered into J
-int launch_fused_tail(rk_world* w, hipStream_t s);
+// cleared), staged current windows gathered into J; one launch for both
+int launch_fused_tail(rk_world* w, bool appends, bool gather, hipStream_t s);
 int verify_fast_division(float cfl, float rcp, uint64_t mismatches[2]);
 int upload_mig_table(rk_world* w);
 int launch_reset_counter(rk_world* w, int which, hipStream_t s);

@@ -1995,7 +1995,9 @@ __device__ inline void gather_row(const Geo& g, const float* __restrict__ stage,
 
 // What follows the fused step in one launch: the blocks of the mailboxes'
 // appends (which wait on memory round trips), then those of the record sets',
-// then those of the gather of the currents, none of which needs another.  All
+// then those of the gather of the currents, none of which needs another (while
+// kernels are timed, the first two and the last in a launch each, under their
+// own categories).  All
 // three counts of blocks but the last are multiples of 8, so a block's place
 // among its kind gives its XCD: a brick's neighbours mostly run on the same one
 // (xcd_brick, as the fused step), so the appends to one destination bin's tail
@@ -2009,7 +2011,7 @@ constexpr int REC_BLOCKS = 128;  // they append only what spilled past full mail
 
 __global__ void __launch_bounds__(WG)
   k_fused_tail(Geo g, SpParams sp, MigPtrs m, uint32_t* counters, uint32_t* ovf, int64_t ovf_cap, int span, int nappend,
-               const float* __restrict__ stage, int64_t stride, float* J0, float* J1, float* J2)
+               int nrec, const float* __restrict__ stage, int64_t stride, float* J0, float* J1, float* J2)
 {
   int i = int(blockIdx.x);
   if(i < nappend) {
@@ -2018,11 +2020,11 @@ __global__ void __launch_bounds__(WG)
     return;
   }
   i -= nappend;
-  if(i < REC_BLOCKS) {
-    append_records(g, sp, m, i, REC_BLOCKS, counters, ovf, ovf_cap);
+  if(i < nrec) {
+    append_records(g, sp, m, i, nrec, counters, ovf, ovf_cap);
     return;
   }
-  i -= REC_BLOCKS;
+  i -= nrec;
   const int rows = g.L[0] * g.L[1], total = (rows + 1) / 2;
   const int xcd = i % 8, q8 = total / 8, r8 = total % 8;
   const int pair = xcd * q8 + min(xcd, r8) + i / 8;
@@ -2520,14 +2522,16 @@ int launch_fused(rk_world* w, hipStream_t s, const WallSet* walls, const rk_refl
   return RK_OK;
 }
 
-int launch_fused_tail(rk_world* w, hipStream_t s)
+int launch_fused_tail(rk_world* w, bool appends, bool gather, hipStream_t s)
 {
   const Geo& g = w->g;
   const int span = xcd_span(g, g.nbricks);
-  const int nappend = int(xcd_grid(g.nbricks, span));  // a multiple of 8
-  const int pairs = (g.L[0] * g.L[1] + 1) / 2;
-  hipLaunchKernelGGL(k_fused_tail, dim3(unsigned(nappend + REC_BLOCKS + pairs)), dim3(WG), 0, s, g, make_sp(w), make_mig(w), w->counters,
-                     w->ovf_list, w->ovf_cap, span, nappend, w->jstage, w->jstage_stride, w->J[0], w->J[1], w->J[2]);
+  const int nappend = appends ? int(xcd_grid(g.nbricks, span)) : 0;  // a multiple of 8
+  const int nrec = appends ? REC_BLOCKS : 0;
+  const int pairs = gather ? (g.L[0] * g.L[1] + 1) / 2 : 0;
+  hipLaunchKernelGGL(k_fused_tail, dim3(unsigned(nappend + nrec + pairs)), dim3(WG), 0, s, g, make_sp(w), make_mig(w),
+                     w->counters, w->ovf_list, w->ovf_cap, span, nappend, nrec, w->jstage, w->jstage_stride, w->J[0],
+                     w->J[1], w->J[2]);
   RK_HIP(hipGetLastError());
   return RK_OK;
 }

@@ -63,3 +63,29 @@ def test_one_lap_parity_share_edges(orc, n, brick, pusher):
     g, o = gpu_fields(grid), w.global_fields()
     assert rel_err(g[0:3], o[0:3]) < 1e-6
     assert rel_err(g[6:9], o[6:9]) < 1e-6
+
+
+def test_timed_step_takes_the_same_work_under_its_categories():
+    # the appends and the gather of the currents share a launch unless kernels
+    # are timed; a cold plasma of a particle per cell has few leavers, so the
+    # gather takes the longer
+    import torch
+    from runko_amd import _lib as L
+    from runko_amd.init import turbulence_world
+    from runko_amd.stepper import BatchedLap
+
+    worlds = [turbulence_world(N=128, tile=32, ppc=1, theta=1e-4, sigma=1e-4, seed=3)[0] for _ in range(2)]
+    laps = [BatchedLap(w) for w in worlds]
+    ms, cnt = np.zeros((2, 9)), np.zeros(9, dtype=np.int64)
+    for rep in range(2):
+        for timed, (w, lap) in enumerate(zip(worlds, laps)):
+            L.check(L.lib().rk_profile_enable(w.h, timed))
+            lap()
+            lap.settle()
+            if timed:
+                L.check(L.lib().rk_profile_read(w.h, ms[rep].ctypes.data, cnt.ctypes.data))
+                L.check(L.lib().rk_profile_enable(w.h, 0))
+        assert torch.equal(worlds[0].F, worlds[1].F)
+        assert worlds[0].total_particles() == worlds[1].total_particles()
+    deposit, append = (dict(zip(L.PROF_CATEGORIES, ms.min(0)))[k] for k in ("deposit", "append"))
+    assert deposit > append > 0, (deposit, append)
