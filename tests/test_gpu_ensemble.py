@@ -41,6 +41,12 @@ UNEVEN = [
     dict(n=(2, 2, 64), charges=[-0.02, 0.02], masses=[1.0, 1.0], counts=[90, 80]),
 ]
 
+# alone a box of 4^3-cell bricks and particle blocks of 256; with the other one
+# bricks of 8^3 and blocks of 8192, or a list of its particles by brick
+SMALL = dict(n=(41, 18, 20), charges=[-0.02, 0.02], masses=[1.0, 1.0], counts=[5000, 4001])
+LONG_BLOCKS = [SMALL, dict(n=(64, 64, 64), charges=[-1e-3, 1e-3], masses=[1.0, 1.0], counts=[4200000, 4200000])]
+LISTED = [SMALL, dict(n=(256, 256, 264), charges=[-0.01], masses=[1.0], counts=[3000])]
+
 
 def build(dtype, seed=3, boxes=BOXES):
     gen = torch.Generator(device="cuda")
@@ -58,8 +64,9 @@ def build(dtype, seed=3, boxes=BOXES):
     return ens, singles, states, cat
 
 
-cases = pytest.mark.parametrize("dtype, boxes", [(torch.float32, BOXES), (torch.float64, BOXES), (torch.float64, UNEVEN)],
-                                ids=["fp32", "fp64", "fp64-uneven"])
+cases = pytest.mark.parametrize("dtype, boxes", [(torch.float32, BOXES), (torch.float64, BOXES), (torch.float64, UNEVEN),
+                                                 (torch.float32, LONG_BLOCKS), (torch.float32, LISTED)],
+                                ids=["fp32", "fp64", "fp64-uneven", "fp32-long-blocks", "fp32-listed"])
 
 
 @cases

@@ -1,9 +1,9 @@
 """Mailbox spills of the fused particle step.
 
 Every brick writes its leavers into its own mailbox; past the mailbox's
-capacity they spill into the shared record sets 0 and 1, which
-k_append_records appends after the mailboxes (and then clears its record
-counters itself).  Two copies of a hot 64^3 turbulence world, one with the
+capacity they spill into the shared record sets 0 and 1, which blocks of
+k_fused_tail append beside those of the mailboxes, in no order (and then clear
+the sets' record counters).  Two copies of a hot 64^3 turbulence world, one with the
 default mailboxes and one with 64 records per brick (about a tenth of a
 brick's leavers per lap here), must stay identical lap for lap: the same
 particles (compared by id) bit for bit, and the same fields bit for bit,

@@ -239,6 +239,7 @@ def test_simulation_io_snapshots(tmp_path):
 @pytest.mark.parametrize("n, stride, nbins, nspecies", [
     ((12, 9, 10), 1, 60, 2),    # bricks of 6 x 1 x 5 cells, coarse cells inside one brick
     ((12, 9, 10), 5, 60, 2),    # coarse cells and x bins shared by bricks, cells past the last one
+    ((12, 9, 10), 11, 60, 2),   # longer than a tile's y and z sides: spectra only, one x bin a tile, cells past it
     ((8, 16, 16), 8, 5000, 2),  # more counters than a workgroup's LDS holds
     ((16, 16, 16), 2, 128, 2),  # several bricks per workgroup (4^3 tiles)
 ])
