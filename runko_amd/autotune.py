@@ -9,8 +9,9 @@ particles per cell and the temperature.  `tune_shape` times the fused
 kernel (HIP events of the library's own profile) for every candidate brick
 shape, and for 8^3 bricks both workgroup sizes (512 and 256 threads), on a
 small periodic world of the same tile size, ppc and theta (2 x 2 x 2 tiles,
-seeded turbulence set-up), and returns the fastest per particle.
-Results are cached per (tile, ppc, theta) for the process.
+seeded turbulence set-up), and returns the fastest per particle, or the
+shape that a world has by default where the trial does not tell them apart
+(`RULE_MARGIN`).  Results are cached per (tile, ppc, theta) for the process.
 
 `tune_fused_launch` picks, on the live world, between the two launch forms
 of the fused step (one workgroup per brick, or persistent workgroups taking
@@ -27,12 +28,19 @@ import numpy as np
 import torch
 
 from . import _lib as L
+from .world import choose_brick
 
 # LDS bytes of one fused workgroup: E/B node means (float, 6 per node over
 # (b + 2)^3) plus the current window (double, 3 per node over (b + 3)^3);
 # at most 64 KiB, so two workgroups share a CU's 160 KiB
 LDS_LIMIT = 64 * 1024
 SIDES = (4, 8, 16)
+# The default shape (choose_brick, 512 threads) is kept unless another takes
+# less than 1 / RULE_MARGIN of its time.  Trials of one shape differ by up to
+# 3 %, and the trial world runs a single round of workgroups: it has 4 x 8 x 16
+# bricks within 1 % of 8^3 (ahead in some runs), which take 3 % longer on 512^3
+# cells (k_fused 98.3 against 95.5 ms).
+RULE_MARGIN = 1.05
 
 _CACHE = {}
 
@@ -94,7 +102,8 @@ def time_brick(tile, brick, ppc, theta, steps=3, warmup=2, seed=1, workgroup=512
 def tune_shape(tile, ppc=16, theta=0.3, candidates=None, steps=3):
     """(best brick, best threads per workgroup, {(brick, threads): ns per
     particle}) for cubic tiles of side `tile`; candidates: (brick, threads)
-    pairs (default candidate_shapes)."""
+    pairs, of which the fastest is best (default candidate_shapes, where the
+    default shape is best unless another is clearly faster)."""
     key = (int(tile), int(ppc), float(theta))
     if key in _CACHE and candidates is None:
         return _CACHE[key]
@@ -108,6 +117,10 @@ def tune_shape(tile, ppc=16, theta=0.3, candidates=None, steps=3):
     if not table:
         raise RuntimeError(f"autotune: no brick shape ran for tile {tile}")
     best = min(table, key=table.get)
+    if candidates is None:
+        rule = (choose_brick((tile,) * 3), 512)
+        if rule in table and table[rule] <= RULE_MARGIN * table[best]:
+            best = rule
     out = (best[0], best[1], table)
     if candidates is None:
         _CACHE[key] = out
@@ -118,11 +131,11 @@ def tune_brick(tile, ppc=16, theta=0.3, candidates=None, steps=3):
     """(best brick, {brick: ns per particle}) for cubic tiles of side `tile`
     (each brick at its best workgroup size); candidates: bricks."""
     pairs = None if candidates is None else [(b, 512) for b in candidates]
-    _, _, table = tune_shape(tile, ppc, theta, pairs, steps)
+    best, _, table = tune_shape(tile, ppc, theta, pairs, steps)
     per = {}
     for (b, _), v in table.items():
         per[b] = min(v, per.get(b, v))
-    return min(per, key=per.get), per
+    return best, per
 
 
 def tune_fused_launch(world, lap, laps_per_mode=1):
