@@ -151,16 +151,17 @@ struct CurlB {
 // workgroups of DWG threads (at most MERGED_BLOCKS of them, see merged()).
 struct BoxGrid {
   int gx, gy, gz, bx, by;
+  int seg;  // workgroups that share a row (few, long rows)
   __host__ __device__ int blocks() const { return gx * gy * gz; }
 };
 struct BoxPlace {
-  int z, i, j, tx;
+  int z, i, j, tx, step;
   bool ok;
 };
 __device__ inline BoxPlace place(const BoxGrid& g, int blk)
 {
   const int tid = int(threadIdx.x), ty = tid / g.bx, x = blk % g.gx, q = blk / g.gx;
-  return BoxPlace {q / g.gy, q % g.gy, x * g.by + ty, tid - ty * g.bx, ty < g.by};
+  return BoxPlace {q / g.gy, q % g.gy, x / g.seg * g.by + ty, x % g.seg * g.bx + tid - ty * g.bx, g.seg * g.bx, ty < g.by};
 }
 
 // the nodes (i, j, k), k = tx, tx + bx, ..., of a box
@@ -389,7 +390,10 @@ __device__ inline Cov covers(const Axis& a, int i)
 // axis) that hold it.  A node lies in at most eight windows as a rule: their
 // loads are issued together, the absent ones on the own window and not added
 // (k_djgather on 96^3 30.8 -> 26.3 us, on 16^3 7.8 -> 4.0 us; a chain of loads before).
-template<class T, int NC, int W>
+// THIRD: bricks of two cells along an axis may put a node in a third window
+// there; then up to three at a time (2 x 2 x 4096 cells, k_dfinish: 196 us in a
+// chain by a workgroup a row, 120 us so, 10 us with sixteen workgroups a row).
+template<class T, int NC, int W, bool THIRD>
 __device__ inline void sum_windows(const DEnt<T>& en, const Cov& ci, const Cov& cj, const Cov& ck,
                                    const T* __restrict__ st, T (&sum)[NC])
 {
@@ -400,7 +404,7 @@ __device__ inline void sum_windows(const DEnt<T>& en, const Cov& ci, const Cov& 
   };
 #pragma unroll
   for(int q = 0; q < NC; ++q) sum[q] = T(0);
-  if(!(ci.both || cj.both || ck.both)) {
+  if(!THIRD || !(ci.both || cj.both || ck.both)) {
     T v[8][NC];
 #pragma unroll
     for(int m = 0; m < 8; ++m) {
@@ -419,19 +423,31 @@ __device__ inline void sum_windows(const DEnt<T>& en, const Cov& ci, const Cov& 
     }
     return;
   }
-  for(int m = 0; m < 27; ++m) {
-    const int o[3] = {m / 9, m / 3 % 3, m % 3};
-    const Cov* c[3] = {&ci, &cj, &ck};
-    bool in = true;
-    for(int a = 0; a < 3; ++a) in = in && (o[a] == 0 || (o[a] == 1 ? c[a]->ok : c[a]->both));
-    if(!in) continue;
-    int br[3], of[3];
-    for(int a = 0; a < 3; ++a) {
-      br[a] = o[a] == 0 ? c[a]->brick[0] : (o[a] == 1 ? c[a]->brick[1] : c[a]->brick[2]);
-      of[a] = o[a] == 0 ? c[a]->off[0] : (o[a] == 1 ? c[a]->off[1] : c[a]->off[2]);
+  if constexpr(THIRD) {
+    auto held = [](const Cov& c, int o) { return o == 0 || (o == 1 ? c.ok : c.both); };
+    auto pick = [](const int (&v)[3], int o) { return o == 0 ? v[0] : (o == 1 ? v[1] : v[2]); };
+#pragma unroll 1
+    for(int m = 0; m < 9; ++m) {
+      const int x = m / 3, y = m % 3;
+      if(!held(ci, x) || !held(cj, y)) continue;
+      const int64_t row = (int64_t(pick(ci.brick, x)) * en.ax[1].nb + pick(cj.brick, y)) * en.ax[2].nb;
+      const int at = (pick(ci.off, x) * W + pick(cj.off, y)) * W;
+      T v[3][NC];
+#pragma unroll
+      for(int z = 0; z < 3; ++z) {
+        const int k = held(ck, z) ? z : 0;
+        const T* w = st + (row + pick(ck.brick, k)) * (NC * V) + at + pick(ck.off, k);
+#pragma unroll
+        for(int q = 0; q < NC; ++q) v[z][q] = w[q * V];
+      }
+#pragma unroll
+      for(int z = 0; z < 3; ++z)
+#pragma unroll
+        for(int q = 0; q < NC; ++q) {
+          const T t = sum[q] + v[z][q];
+          sum[q] = held(ck, z) ? t : sum[q];
+        }
     }
-    const T* w = st + ((int64_t(br[0]) * en.ax[1].nb + br[1]) * en.ax[2].nb + br[2]) * (NC * V) + (of[0] * W + of[1]) * W + of[2];
-    for(int q = 0; q < NC; ++q) sum[q] += w[q * V];
   }
 }
 
@@ -450,7 +466,7 @@ __device__ inline void mgather_row(const DEnt<T>& en, G3<T> LE, G3<T> LB, G3<T> 
   for(int k = tx; k < b.n[2]; k += bx) {
     const Cov ck = covers<1, 1>(en.ax[2], k);
     T s[6];
-    sum_windows<T, 6, W>(en, ci, cj, ck, mst, s);
+    sum_windows<T, 6, W, false>(en, ci, cj, ck, mst, s);
     const int64_t c = en.c0 + cidx(b.n, i, j, k);
 #pragma unroll
     for(int q = 0; q < 3; ++q) {
@@ -484,7 +500,7 @@ __device__ inline void jgather_row(const DEnt<T>& en, G3<T> J, const T* __restri
   for(int k = tx; k < b.n[2]; k += bx) {
     const Cov ck = covers<1, 2>(en.ax[2], k);
     T s[3];
-    sum_windows<T, 3, D>(en, ci, cj, ck, jst, s);
+    sum_windows<T, 3, D, true>(en, ci, cj, ck, jst, s);
     const int64_t c = cidx(b.n, i, j, k);
 #pragma unroll
     for(int q = 0; q < 3; ++q) J.c[q][c] += s[q];
@@ -1003,7 +1019,7 @@ __global__ void __launch_bounds__(DWG)
   blk -= pblocks;
   const bool second = blk >= bg.blocks();
   const BoxPlace pl = place(bg, second ? blk - bg.blocks() : blk);
-  if(pl.ok) curl_b_row(tab[pl.z], second ? c2 : c1, pl.i, pl.j, pl.tx, bg.bx);
+  if(pl.ok) curl_b_row(tab[pl.z], second ? c2 : c1, pl.i, pl.j, pl.tx, pl.step);
 }
 
 // After it, the particles back into their order and the gather of the bricks'
@@ -1021,8 +1037,8 @@ __global__ void __launch_bounds__(DWG)
   }
   const BoxPlace pl = place(bg, blk - pblocks);
   if(!pl.ok) return;
-  if constexpr(ADJ) mgather_row<T, BR>(tab[pl.z], F, LB, LBout, st, pl.i, pl.j, pl.tx, bg.bx);
-  else jgather_row<T, BR>(tab[pl.z], F, st, pl.i, pl.j, pl.tx, bg.bx);
+  if constexpr(ADJ) mgather_row<T, BR>(tab[pl.z], F, LB, LBout, st, pl.i, pl.j, pl.tx, pl.step);
+  else jgather_row<T, BR>(tab[pl.z], F, st, pl.i, pl.j, pl.tx, pl.step);
 }
 
 // one brick of a box
@@ -1830,7 +1846,10 @@ int unsort_particles(const DiffImpl& h, int which, G3<T> x, G3<T> u, hipStream_t
 inline BoxGrid box_grid(const DiffImpl& h)
 {
   const dim3 g = grid_of(h), b = block_of(h);
-  return BoxGrid {int(g.x), int(g.y), int(g.z), int(b.x), int(b.y)};
+  // a row longer than a workgroup is shared while there are fewer rows than CUs
+  const int64_t blocks = int64_t(g.x) * g.y * g.z;
+  const int seg = blocks < 256 ? (h.nmax[2] + int(b.x) - 1) / int(b.x) : 1;
+  return BoxGrid {int(g.x) * seg, int(g.y), int(g.z), int(b.x), int(b.y), seg};
 }
 
 // Launches are merged where they bound the step: particle blocks of DWG threads

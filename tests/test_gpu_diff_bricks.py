@@ -34,6 +34,7 @@ def random_state(n, counts, seed):
 
 @pytest.mark.parametrize("n, counts, cfl", [
     ((2, 3, 5), (40, 23), 0.45),            # sides shorter than a brick: windows wrap onto themselves
+    ((2, 5, 700), (300, 200), 0.45),        # nodes in three windows; rows shared by three workgroups
     ((5, 9, 17), (700, 901), 0.45),         # ragged bricks of at most 4 cells, 7 blocks of 256 particles
     ((6, 5, 9), (257, 1), 1.4),             # moves beyond the neighbouring cell
     ((41, 18, 20), (70001, 70000), 0.45),   # blocks of 1024 particles
@@ -72,29 +73,39 @@ def test_listed_particles_in_cell_order():
     check_step(n, counts, 0.45, (E, B, x, u))
 
 
+def milliseconds(box, n_particles, n, shape, adjoint=True, passes=4):
+    g = torch.Generator(device=DEV)
+    g.manual_seed(2)
+    hi = torch.tensor(n, device=DEV, dtype=torch.float32).view(3, 1)
+    s = (0.05 * torch.randn(shape, generator=g, device=DEV), 0.05 * torch.randn(shape, generator=g, device=DEV),
+         (torch.rand((3, n_particles), generator=g, device=DEV) * hi * 0.999999).contiguous(),
+         torch.randn((3, n_particles), generator=g, device=DEV))
+    out, times = box.empty_state(), []
+    for _ in range(passes):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        box.step(s, out)
+        if adjoint:
+            box.step_adjoint(s, s, out)
+        b.record()
+        torch.cuda.synchronize()
+        times.append(a.elapsed_time(b))
+    assert box.error_count() == 0
+    return min(times)
+
+
+def test_long_rows_cost_what_short_rows_cost():
+    # a box of 2 x 2 x 4096 cells against the same lying along x: the nodes'
+    # three windows in a chain, by four workgroups, took 3.5 times as long
+    t = [milliseconds(DiffBox(n, Q, M, (20000, 20000)), 40000, n, (3,) + n, adjoint=False, passes=30)
+         for n in ((2, 2, 4096), (4096, 2, 2))]
+    assert t[0] < 2 * t[1], t
+
+
 def test_many_bricks_cost_what_their_parts_cost():
     # a box of 262144 bricks against 16 boxes of 16384 with the same cells and
     # particles in all: walking the runs of groups of 4^3 bricks took 2.6 times
     # as long (61 against 24 ms), the list takes 1.1 times
-    def milliseconds(box, n_particles, n, shape):
-        g = torch.Generator(device=DEV)
-        g.manual_seed(2)
-        hi = torch.tensor(n, device=DEV, dtype=torch.float32).view(3, 1)
-        s = (0.05 * torch.randn(shape, generator=g, device=DEV), 0.05 * torch.randn(shape, generator=g, device=DEV),
-             (torch.rand((3, n_particles), generator=g, device=DEV) * hi * 0.999999).contiguous(),
-             torch.randn((3, n_particles), generator=g, device=DEV))
-        out, times = box.empty_state(), []
-        for _ in range(4):
-            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
-            a.record()
-            box.step(s, out)
-            box.step_adjoint(s, s, out)
-            b.record()
-            torch.cuda.synchronize()
-            times.append(a.elapsed_time(b))
-        assert box.error_count() == 0
-        return min(times)
-
     whole, part, k = (2, 4096, 4096), (2, 1024, 1024), 1 << 24
     one = milliseconds(DiffBox(whole, Q, M, (k, k)), 2 * k, whole, (3,) + whole)
     parts = DiffEnsemble([dict(n=part, charges=Q, masses=M, counts=(k // 16, k // 16))] * 16)
