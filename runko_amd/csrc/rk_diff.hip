@@ -1168,8 +1168,9 @@ struct Runs {
 // scanned NT at a time; a thread takes a contiguous share of the records they
 // hold, so neighbouring lanes are far apart in a run (the particles of a cell
 // that lie one after the other go to one lane, and the lanes' LDS adds to
-// different nodes).  body(record, its place).
-template<class T, int NT, bool LIST, class Body>
+// different nodes).  body(record, its place).  SPLIT: the gridDim.y workgroups of
+// a brick take a share of the rows each.
+template<class T, int NT, bool LIST, bool SPLIT, class Body>
 __device__ inline void for_records(const DEnt<T>& en, const Runs& runs, int64_t k, const Rec<T>* A, Body&& body)
 {
   const int tid = int(threadIdx.x);
@@ -1198,9 +1199,11 @@ __device__ inline void for_records(const DEnt<T>& en, const Runs& runs, int64_t 
   const int64_t P = runs.P;
   const uint16_t* tabl = reinterpret_cast<const uint16_t*>(runs.rows + en.row0) + k;
   const int64_t stride = 2 * int64_t(en.rowlen);
-  for(int64_t r0 = 0; r0 < en.nrow; r0 += NT) {
+  const int64_t ra = SPLIT ? en.nrow * blockIdx.y / gridDim.y : 0;
+  const int64_t rb = SPLIT ? en.nrow * (blockIdx.y + 1) / gridDim.y : en.nrow;
+  for(int64_t r0 = ra; r0 < rb; r0 += NT) {
     uint32_t a = 0, len = 0;
-    if(r0 + tid < en.nrow) {
+    if(r0 + tid < rb) {
       const uint16_t* e = tabl + (r0 + tid) * stride;
       a = e[0];
       len = e[1] - a;
@@ -1272,13 +1275,34 @@ __device__ __attribute__((noinline)) void deposit_far(const DBox<T>& b, T* J0, T
       if(zig_has(m, c)) atomic_add(&J[c][box_node(b, k, ZOFF[m])], v[m][c]);
 }
 
+// a split brick's window as one of its workgroups summed it
+template<int N, int NT>
+__device__ inline void store_part(double* __restrict__ part, const double (&win)[N])
+{
+  double* p = part + (int64_t(blockIdx.x) * gridDim.y + blockIdx.y) * N;
+  for(int q = int(threadIdx.x); q < N; q += NT) p[q] = win[q];
+}
+
+// their sum, brick blockIdx.x
+template<int N, int NT>
+__device__ inline void sum_parts(const double* __restrict__ part, int split, double (&win)[N])
+{
+  const double* p = part + int64_t(blockIdx.x) * split * N;
+  for(int q = int(threadIdx.x); q < N; q += NT) {
+    double v = 0.0;
+#pragma unroll 8
+    for(int k = 0; k < split; ++k) v += p[int64_t(k) * N + q];
+    win[q] = v;
+  }
+}
+
 // the forward step of one brick's particles; results replace the records (a
 // second set of records made the step 12 to 35 % slower: twice the lines to
 // hold in cache)
 template<class T, int BR, int NT, bool LIST>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 5 : 4)))
   k_dstep(const DEnt<T>* __restrict__ tab, const uint16_t* __restrict__ kmap, G3<T> E, G3<T> B,
-          Runs runs, Rec<T>* A, T* __restrict__ jst, G3<T> J)
+          Runs runs, Rec<T>* A, T* __restrict__ jst, G3<T> J, double* __restrict__ part)
 {
   constexpr int M = BR + 1, D = BR + 3, V = D * D * D;
   __shared__ double win[3 * V];
@@ -1293,7 +1317,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(
   for(int q = int(threadIdx.x); q < 3 * V; q += NT) win[q] = 0.0;
   stage_nodes<T, BR, NT>(b, bk, E, B, nm);
   __syncthreads();
-  for_records<T, NT, LIST>(en, runs, kb, A, [&](Rec<T> r, int64_t at) {
+  for_records<T, NT, LIST, BR == 4>(en, runs, kb, A, [&](Rec<T> r, int64_t at) {
     Fwd<T> f;
     int cell[3], l[3];
 #pragma unroll
@@ -1348,8 +1372,24 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(
     }
   });
   __syncthreads();
+  if constexpr(BR == 4)
+    if(gridDim.y > 1) {
+      store_part<3 * V, NT>(part, win);
+      return;
+    }
   T* w = jst + int64_t(blockIdx.x) * (3 * V);
   for(int q = int(threadIdx.x); q < 3 * V; q += NT) w[q] = T(win[q]);
+}
+
+// split bricks: their current windows
+template<class T, int BR, int NT>
+__global__ void __launch_bounds__(NT) k_dstep_sum(const double* __restrict__ part, int split, T* __restrict__ jst)
+{
+  constexpr int N = 3 * (BR + 3) * (BR + 3) * (BR + 3);
+  __shared__ double win[N];
+  sum_parts<N, NT>(part, split, win);
+  T* w = jst + int64_t(blockIdx.x) * N;
+  for(int q = int(threadIdx.x); q < N; q += NT) w[q] = T(win[q]);  // (each thread its own)
 }
 
 // gathered adjoint of one zigzag segment: dL/dF and dL/dW (per axis); L(d, o)
@@ -1395,6 +1435,35 @@ __device__ inline void cross_adj(const T a[3], const T b[3], const T gc[3], T ga
   for(int k = 0; k < 3; ++k) gb[k] += t[k];
 }
 
+// a brick's window of field adjoints from its node-mean adjoints mw
+template<class T, int BR, int NT>
+__device__ inline void store_means(const BrickOf& bk, const double* mw, T* __restrict__ mst)
+{
+  constexpr int M = BR + 1, MV = M * M * M;
+  // node means back to the staggered components.  E_x(node N) = (Ex[N-x] +
+  // Ex[N]) / 2, so Ex[n] receives (ME_x[n] + ME_x[n+x]) / 2; B_x(node N) =
+  // (Bx[N] + Bx[N-y] + Bx[N-z] + Bx[N-y-z]) / 4, so Bx[n] receives the mean of
+  // MB_x over n, n+y, n+z, n+y+z: a window of one node before the brick to one after
+  constexpr int W = BR + 2, WV = W * W * W;
+  T* out = mst + int64_t(blockIdx.x) * (6 * WV);
+  for(int q = int(threadIdx.x); q < WV; q += NT) {
+    const int o[3] = {q / (W * W) - 1, q / W % W - 1, q % W - 1};
+    auto at = [&](int c, int x, int y, int z) {
+      const int p[3] = {o[0] + x, o[1] + y, o[2] + z};
+#pragma unroll
+      for(int a = 0; a < 3; ++a)
+        if(p[a] < 0 || p[a] > bk.n[a]) return 0.0;
+      return mw[c * MV + (p[0] * M + p[1]) * M + p[2]];
+    };
+    out[q] = T((at(0, 0, 0, 0) + at(0, 1, 0, 0)) * 0.5);
+    out[WV + q] = T((at(1, 0, 0, 0) + at(1, 0, 1, 0)) * 0.5);
+    out[2 * WV + q] = T((at(2, 0, 0, 0) + at(2, 0, 0, 1)) * 0.5);
+    out[3 * WV + q] = T(((at(3, 0, 0, 0) + at(3, 0, 1, 0)) + (at(3, 0, 0, 1) + at(3, 0, 1, 1))) * 0.25);
+    out[4 * WV + q] = T(((at(4, 0, 0, 0) + at(4, 1, 0, 0)) + (at(4, 0, 0, 1) + at(4, 1, 0, 1))) * 0.25);
+    out[5 * WV + q] = T(((at(5, 0, 0, 0) + at(5, 1, 0, 0)) + (at(5, 0, 1, 0) + at(5, 1, 1, 0))) * 0.25);
+  }
+}
+
 // the adjoint of one brick's particles.  L: the filtered adjoint of E', whose
 // negative is the adjoint of J.  Each particle recomputes its forward step,
 // applies the chain rule by hand and adds its node-mean adjoints (dL/dE, dL/dB
@@ -1404,7 +1473,8 @@ __device__ inline void cross_adj(const T a[3], const T b[3], const T gc[3], T ga
 template<class T, int BR, int NT, bool LIST>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 2)))
   k_dadj(const DEnt<T>* __restrict__ tab, const uint16_t* __restrict__ kmap, G3<T> E, G3<T> B, G3<T> L,
-         Runs runs, const Rec<T>* __restrict__ A, Rec<T>* __restrict__ lam, T* __restrict__ mst)
+         Runs runs, const Rec<T>* __restrict__ A, Rec<T>* __restrict__ lam, T* __restrict__ mst,
+         double* __restrict__ part)
 {
   constexpr int M = BR + 1, MV = M * M * M, D = BR + 3, V = D * D * D;
   __shared__ double mw[6 * MV];
@@ -1431,7 +1501,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(
   }
   __syncthreads();
   const T cfl = b.cfl;
-  for_records<T, NT, LIST>(en, runs, kb, A, [&](const Rec<T>& r, int64_t at) {
+  for_records<T, NT, LIST, BR == 4>(en, runs, kb, A, [&](const Rec<T>& r, int64_t at) {
     Rec<T> g = lam[at];
     Fwd<T> f;
     int cell[3], l[3];
@@ -1567,28 +1637,26 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(
     lam[at] = g;
   });
   __syncthreads();
-  // node means back to the staggered components.  E_x(node N) = (Ex[N-x] +
-  // Ex[N]) / 2, so Ex[n] receives (ME_x[n] + ME_x[n+x]) / 2; B_x(node N) =
-  // (Bx[N] + Bx[N-y] + Bx[N-z] + Bx[N-y-z]) / 4, so Bx[n] receives the mean of
-  // MB_x over n, n+y, n+z, n+y+z: a window of one node before the brick to one after
-  constexpr int W = BR + 2, WV = W * W * W;
-  T* out = mst + int64_t(blockIdx.x) * (6 * WV);
-  for(int q = int(threadIdx.x); q < WV; q += NT) {
-    const int o[3] = {q / (W * W) - 1, q / W % W - 1, q % W - 1};
-    auto at = [&](int c, int x, int y, int z) {
-      const int p[3] = {o[0] + x, o[1] + y, o[2] + z};
-#pragma unroll
-      for(int a = 0; a < 3; ++a)
-        if(p[a] < 0 || p[a] > bk.n[a]) return 0.0;
-      return mw[c * MV + (p[0] * M + p[1]) * M + p[2]];
-    };
-    out[q] = T((at(0, 0, 0, 0) + at(0, 1, 0, 0)) * 0.5);
-    out[WV + q] = T((at(1, 0, 0, 0) + at(1, 0, 1, 0)) * 0.5);
-    out[2 * WV + q] = T((at(2, 0, 0, 0) + at(2, 0, 0, 1)) * 0.5);
-    out[3 * WV + q] = T(((at(3, 0, 0, 0) + at(3, 0, 1, 0)) + (at(3, 0, 0, 1) + at(3, 0, 1, 1))) * 0.25);
-    out[4 * WV + q] = T(((at(4, 0, 0, 0) + at(4, 1, 0, 0)) + (at(4, 0, 0, 1) + at(4, 1, 0, 1))) * 0.25);
-    out[5 * WV + q] = T(((at(5, 0, 0, 0) + at(5, 1, 0, 0)) + (at(5, 0, 1, 0) + at(5, 1, 1, 0))) * 0.25);
-  }
+  if constexpr(BR == 4)
+    if(gridDim.y > 1) {
+      store_part<6 * MV, NT>(part, mw);
+      return;
+    }
+  store_means<T, BR, NT>(bk, mw, mst);
+}
+
+// split bricks: their windows of field adjoints
+template<class T, int BR, int NT>
+__global__ void __launch_bounds__(NT)
+  k_dadj_sum(const DEnt<T>* __restrict__ tab, const uint16_t* __restrict__ kmap, const double* __restrict__ part, int split,
+             T* __restrict__ mst)
+{
+  constexpr int MV = (BR + 1) * (BR + 1) * (BR + 1);
+  __shared__ double mw[6 * MV];
+  const DEnt<T>& en = tab[kmap[blockIdx.x]];
+  sum_parts<6 * MV, NT>(part, split, mw);
+  __syncthreads();
+  store_means<T, BR, NT>(brick_of_box(en, int64_t(blockIdx.x) - en.k0), mw, mst);
 }
 
 }  // namespace
@@ -1618,6 +1686,8 @@ struct DiffImpl {
   uint32_t* bstart = nullptr;        // listed: the bricks' starts in it
   uint32_t* bsums = nullptr;         // listed: sums of SCAN counters each
   void* stage = nullptr;             // per brick: its current or node-mean adjoint window
+  int split = 1;                     // workgroups of a brick
+  double* part = nullptr;            // split bricks: the window of each of their workgroups
   unsigned long long* err = nullptr;
 };
 
@@ -1657,6 +1727,12 @@ constexpr int GROUPS_MAX = 32000;
 
 // Layout of the particle phase.
 //  * Bricks of 8 cells per axis, of 4 while those are fewer than one per CU.
+//  * Bricks of 4 cells that are few and full are split over workgroups, a share
+//    of the rows each, until there are two per CU or 1024 records for each.  One
+//    workgroup a brick left the chip idle, below the particle kernels before
+//    bricks: 4^3 cells with 2e5 particles, adjoint 3.48 ms (2.05 ms before), 0.14
+//    ms so; 8^3 with 2e5 0.51 (0.39), 0.08; with 2e4 0.084, 0.062 (4096 records each:
+//    0.14 and 0.084 ms).
 //  * A particle block is as long as keeps two and more blocks per CU busy: its
 //    runs (P / bricks records of a mixed box) are what a brick reads in one
 //    piece.  2.8e7 mixed particles, P = 4096 and 8192: k_dbin<adjoint> + k_dadj
@@ -1715,6 +1791,12 @@ hipError_t upload_table(DiffImpl& h)
   if(e == hipSuccess) e = put(&h.kmap, km);
   const size_t win = size_t(6) * (h.br + 2) * (h.br + 2) * (h.br + 2);  // the larger of the two windows
   if(e == hipSuccess) e = hipMalloc(&h.stage, h.vb * win * size_t(h.nbricks));
+  if(h.br == 4) {
+    h.split = int(std::clamp<int64_t>(std::min(np / (h.nbricks * 1024), 512 / h.nbricks), 1, 64));
+    // doubles of the larger of the two windows as they are summed
+    if(h.split > 1 && e == hipSuccess)
+      e = hipMalloc(reinterpret_cast<void**>(&h.part), sizeof(double) * 3 * 7 * 7 * 7 * size_t(h.nbricks) * size_t(h.split));
+  }
   const size_t n1 = size_t(std::max<int64_t>(np, 1));
   for(int i = 0; i < 2 && e == hipSuccess; ++i) e = hipMalloc(&h.recs[i], sizeof(Rec<T>) * n1);
   if(e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&h.slot), sizeof(uint16_t) * n1);
@@ -1908,11 +1990,16 @@ int step_t(DiffImpl& h, const rk_diff_state* in, rk_diff_state* out, hipStream_t
     constexpr int NT = brick_threads(BR);
     T* jst = static_cast<T*>(h.stage);
     auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, dim3(unsigned(h.nbricks)), dim3(NT), 0, st, b, h.kmap, E, B1, runs_of(h),
-                         static_cast<Rec<T>*>(h.recs[0]), jst, J);
+      hipLaunchKernelGGL(kern, dim3(unsigned(h.nbricks), unsigned(h.split)), dim3(NT), 0, st, b, h.kmap, E, B1, runs_of(h),
+                         static_cast<Rec<T>*>(h.recs[0]), jst, J, h.part);
     };
     h.listed ? go(k_dstep<T, BR, NT, BR == 8>) : go(k_dstep<T, BR, NT, false>);  // (listed boxes have bricks of 8 cells)
     RK_HIP(hipGetLastError());
+    if constexpr(BR == 4)
+      if(h.split > 1) {
+        hipLaunchKernelGGL((k_dstep_sum<T, BR, NT>), dim3(unsigned(h.nbricks)), dim3(NT), 0, st, h.part, h.split, jst);
+        RK_HIP(hipGetLastError());
+      }
     if(merged(h)) {
       const BoxGrid bg = box_grid(h);
       hipLaunchKernelGGL((k_dfinish<T, BR, false>), dim3(unsigned(h.pblocks + bg.blocks())), dim3(DWG), 0, st, b, h.pmap,
@@ -1960,11 +2047,16 @@ int adjoint_t(DiffImpl& h, const rk_diff_state* in, const rk_diff_state* ao, rk_
     constexpr int NT = brick_threads(BR);
     T* mst = static_cast<T*>(h.stage);
     auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, dim3(unsigned(h.nbricks)), dim3(NT), 0, st, b, h.kmap, E, B1, lj, runs_of(h),
-                         static_cast<const Rec<T>*>(h.recs[0]), static_cast<Rec<T>*>(h.recs[1]), mst);
+      hipLaunchKernelGGL(kern, dim3(unsigned(h.nbricks), unsigned(h.split)), dim3(NT), 0, st, b, h.kmap, E, B1, lj,
+                         runs_of(h), static_cast<const Rec<T>*>(h.recs[0]), static_cast<Rec<T>*>(h.recs[1]), mst, h.part);
     };
     h.listed ? go(k_dadj<T, BR, NT, BR == 8>) : go(k_dadj<T, BR, NT, false>);
     RK_HIP(hipGetLastError());
+    if constexpr(BR == 4)
+      if(h.split > 1) {
+        hipLaunchKernelGGL((k_dadj_sum<T, BR, NT>), dim3(unsigned(h.nbricks)), dim3(NT), 0, st, b, h.kmap, h.part, h.split, mst);
+        RK_HIP(hipGetLastError());
+      }
     // node-mean adjoints: lambda_E += NM_E^T(ME), lambda_B = lambda_B1 = LB2 + NM_B^T(MB)
     LB1 = g3<T>(ai->B);
     if(merged(h)) {
@@ -2075,7 +2167,7 @@ int rk_diff_destroy(rk_diff* h)
       if(p) (void)hipFree(p);
   for(void* q : {h->recs[0], h->recs[1], static_cast<void*>(h->slot), static_cast<void*>(h->rows),
                  static_cast<void*>(h->rank), static_cast<void*>(h->order), static_cast<void*>(h->bstart),
-                 static_cast<void*>(h->bsums), h->stage, static_cast<void*>(h->err), h->tab, static_cast<void*>(h->pmap),
+                 static_cast<void*>(h->bsums), h->stage, static_cast<void*>(h->part), static_cast<void*>(h->err), h->tab, static_cast<void*>(h->pmap),
                  static_cast<void*>(h->kmap)})
     if(q) (void)hipFree(q);
   delete h;

@@ -35,6 +35,8 @@ def random_state(n, counts, seed):
 @pytest.mark.parametrize("n, counts, cfl", [
     ((2, 3, 5), (40, 23), 0.45),            # sides shorter than a brick: windows wrap onto themselves
     ((2, 5, 700), (300, 200), 0.45),        # nodes in three windows; rows shared by three workgroups
+    ((4, 4, 3), (9000, 8001), 0.45),        # one brick, split over 16 workgroups
+    ((8, 7, 5), (20000, 20001), 1.4),       # 8 bricks split over 4, moves beyond the neighbouring cell
     ((5, 9, 17), (700, 901), 0.45),         # ragged bricks of at most 4 cells, 7 blocks of 256 particles
     ((6, 5, 9), (257, 1), 1.4),             # moves beyond the neighbouring cell
     ((41, 18, 20), (70001, 70000), 0.45),   # blocks of 1024 particles
@@ -100,6 +102,13 @@ def test_long_rows_cost_what_short_rows_cost():
     t = [milliseconds(DiffBox(n, Q, M, (20000, 20000)), 40000, n, (3,) + n, adjoint=False, passes=30)
          for n in ((2, 2, 4096), (4096, 2, 2))]
     assert t[0] < 2 * t[1], t
+
+
+def test_few_full_bricks_fill_the_chip():
+    # 8^3 cells with 1e6 particles against 64^3 with as many: one workgroup a brick
+    # took 15 times as long
+    t = [milliseconds(DiffBox(n, Q, M, (500000, 500000)), 1000000, n, (3,) + n, passes=8) for n in ((8, 8, 8), (64, 64, 64))]
+    assert t[0] < 3 * t[1], t
 
 
 def test_many_bricks_cost_what_their_parts_cost():

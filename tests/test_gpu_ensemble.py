@@ -45,6 +45,8 @@ UNEVEN = [
 # bricks of 8^3 and blocks of 8192, or a list of its particles by brick
 SMALL = dict(n=(41, 18, 20), charges=[-0.02, 0.02], masses=[1.0, 1.0], counts=[5000, 4001])
 LONG_BLOCKS = [SMALL, dict(n=(64, 64, 64), charges=[-1e-3, 1e-3], masses=[1.0, 1.0], counts=[4200000, 4200000])]
+SPLIT = [dict(n=(4, 4, 4), charges=[-0.02, 0.02], masses=[1.0, 1.0], counts=[10000, 9000]),  # bricks split over 9 workgroups
+         dict(n=(4, 3, 4), charges=[-0.02], masses=[1.0], counts=[100])]  # alone not split, here rows for one of nine
 LISTED = [SMALL, dict(n=(256, 256, 264), charges=[-0.01], masses=[1.0], counts=[3000])]
 
 
@@ -65,8 +67,8 @@ def build(dtype, seed=3, boxes=BOXES):
 
 
 cases = pytest.mark.parametrize("dtype, boxes", [(torch.float32, BOXES), (torch.float64, BOXES), (torch.float64, UNEVEN),
-                                                 (torch.float32, LONG_BLOCKS), (torch.float32, LISTED)],
-                                ids=["fp32", "fp64", "fp64-uneven", "fp32-long-blocks", "fp32-listed"])
+                                                 (torch.float32, LONG_BLOCKS), (torch.float32, LISTED), (torch.float64, SPLIT)],
+                                ids=["fp32", "fp64", "fp64-uneven", "fp32-long-blocks", "fp32-listed", "fp64-split"])
 
 
 @cases
