@@ -8,12 +8,14 @@
 //                 Boris: u', x' = x + cfl u'/gamma'  pic/particle_boris.h:15-62
 //                 x'' = periodic wrap of x'          pic/tile_communication.c++:98-117
 //                 zigzag deposit of (x'', u') -> J   pic/particle_current_zigzag_1st.c++:225-339
-//   Jf = binomial2^P(J) (periodic, 27 taps)         emf/yee_lattice_current_filter_binomial2.c++:23-76
+//   Jf = binomial2^P(J) (periodic)                  emf/yee_lattice_current_filter_binomial2.c++:23-76
 //   B2 = B1 + (cfl/2) curlE(E)
 //   E' = E + cfl curlB(B2) - Jf                     emf/yee_lattice_fdtd2.c++:68-111, yee_lattice.c++:170-179
 // On a periodic box the tile halos, J_exchange and the copies between filter
-// passes reduce to periodic indexing, so a step gives the tile path's values
-// (J up to the order of its float sums).
+// passes reduce to periodic indexing, so a step gives the tile path's particles
+// bit for bit and its J up to rounding: of the order of the deposit's sums, and
+// of the filter, whose passes are summed axis by axis (k_dfilter) instead of as
+// the reference's 27 taps.
 //
 // Adjoint.  Vector-Jacobian products of each stage, in reverse order.  The
 // discrete curls are negative transposes of each other (curlE^T = -curlB),
@@ -241,7 +243,12 @@ __global__ void __launch_bounds__(DWG)
 
 // R binomial2 passes (yee_lattice_current_filter_binomial2.c++:23-76) of a
 // periodic box in one pass over memory: the passes are separable and commute,
-// so together they are (2R+1)-tap binomials along z, y and x.  A workgroup
+// so together they are (2R+1)-tap binomials along z, y and x.  That is another
+// rounding than the reference's 27 taps a pass, whose weights are powers of two
+// (products with 6, 15 and 20 sixty-fourths round, so they are fused with their
+// sums), and no worse: three FP32 passes against 64 bits 7.6e-8 on a current (27
+// taps 9.3e-8; unfused 8.3e-8), 8.9e-8 on noise, as an adjoint may be (9.4e-8;
+// 9.8e-8).  A workgroup
 // owns FY x FZ columns of nodes of one component and marches over xseg planes:
 // each arriving plane is staged in LDS with R nodes around the tile, summed
 // along z (four nodes a thread, which share their reads) and then along y (four
@@ -265,13 +272,16 @@ __device__ constexpr Taps<T, R> taps()
   else return {{T(1. / 4.), T(2. / 4.)}};
 }
 
+__device__ inline float fused(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ inline double fused(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
 template<class T, int R, int N>
 __device__ inline T tap_sum(const T (&v)[N], int o)
 {
   constexpr Taps<T, R> t = taps<T, R>();
   T s = t.w[R] * v[o + R];
 #pragma unroll
-  for(int k = R - 1; k >= 0; --k) s = s + t.w[k] * (v[o + k] + v[o + 2 * R - k]);
+  for(int k = R - 1; k >= 0; --k) s = fused(t.w[k], v[o + k] + v[o + 2 * R - k], s);
   return s;
 }
 
@@ -1856,7 +1866,10 @@ template<class T>
 int filter_passes(const DiffImpl& h, const DEnt<T>* b, G3<T>& f, hipStream_t st)
 {
   int o = f.c[0] == g3s<T>(h, S_J).c[0] ? S_JT : S_J;
-  // x segments as long as leaves two workgroups per CU: a segment reads 2R planes more than it writes
+  // x segments as long as leaves 512 workgroups a component, six per CU in all (a
+  // segment reads 2R planes more than it writes).  With 256, 512 and 1024: 64^3
+  // 12.6, 13.9 and 14.0 us, 96^3 22.0, 20.8 and 27.9, 128^3 43.6, 32.6 and 43.2;
+  // below 64^3 all within 0.4 us
   const int tz = (h.nmax[2] + FZ - 1) / FZ, cols = tz * ((h.nmax[1] + FY - 1) / FY);
   int xseg = h.nmax[0];
   while(xseg > 2 && int64_t(cols) * ((h.nmax[0] + xseg - 1) / xseg) * int64_t(h.boxes.size()) < 512) xseg = (xseg + 1) / 2;

@@ -122,6 +122,19 @@ def test_many_bricks_cost_what_their_parts_cost():
     assert one < 2 * many, (one, many)
 
 
+def test_filter_rounds_no_more_than_the_27_taps():
+    # from zero fields E' is minus the current, filtered or not: three FP32
+    # passes against 64 bits, and against the reference's 27 taps a pass in FP32
+    n, counts = (40, 36, 44), (60000, 60000)
+    E, _, x, u = (t.to(torch.float32) for t in random_state(n, counts, seed=13))
+    zero = torch.zeros_like(E)
+    J, got = (-DiffBox(n, Q, M, counts, filter_passes=p).step((zero, zero, x, u))[0] for p in (0, 3))
+    exact, taps = J.double(), J
+    for _ in range(3):
+        exact, taps = tp.binomial2(exact), tp.binomial2(taps)
+    assert rel(got.double(), exact) <= rel(taps.double(), exact)
+
+
 def test_segments_several_boxes_away():
     # up to 5.5 cells a step along a side of 2: the current's cells lie up to
     # three sides from the box
