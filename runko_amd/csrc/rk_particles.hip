@@ -310,7 +310,12 @@ __device__ inline float div_cfl(const Geo& g, float x)
   return FAST > 0 ? ieee_div(x, g.cfl) : x / g.cfl;
 }
 
-// x / cfl of a vector: one range check for its three components
+// x / cfl of a vector: one range check for its three components.  A vector with
+// a zero component (fields in a plane, momenta in one) takes the divisions
+// themselves for all three; those calls are not what bounds the step: 64^3, 32
+// particles per cell in a uniform field, all components 242 us, B along z only
+// 242, momenta in the plane too 230 (a check per component: 274, 277 and 265,
+// with the block-wide scan).
 template<int FAST = 0>
 __device__ inline void div_cfl3(const Geo& g, const float x[3], float q[3])
 {
@@ -1607,8 +1612,10 @@ __device__ __forceinline__ void fused_brick(const Geo& g, const SpParams& sp, co
   // registers), so no barrier and no block-wide scan runs in the particle
   // loop, and the waves drift apart: the gathers and current adds of some
   // overlap the arithmetic of others.  The gaps at the ends of the shares are
-  // closed afterwards (below).  VALU issue bounds the loop (88 % busy at 256^3,
-  // 32 particles per cell).  Against a block-wide scan of every 512-particle
+  // closed afterwards (below).  VALU issue bounds the loop (89 % busy at 512^3,
+  // 32 particles per cell; 52 % of the instructions are FP32 arithmetic, 25 %
+  // integer and conversions, the rest moves, compares and lane reads).  Against a
+  // block-wide scan of every 512-particle
   // chunk with a barrier each: 256^3 12.56 -> 11.98 ms, 64^3 128 -> 120 us,
   // with the classification by brick faces and the shorter exact forms.
   constexpr int NW = WGS / 64;
@@ -2208,9 +2215,12 @@ __global__ void __launch_bounds__(WG)
 // workgroup takes 64 particles, a lane each, and its waves count through the
 // tile's ids in LDS, a quarter each.  One launch; a bin-order copy, a library
 // sort and three permutations took eight launches and copies.  Reading the
-// positions of 2048 particles to the host: 212 us that way, 46 us so; of 5000
-// (6528 slots) 203 and 64 us.
-// For up to READBACK_MAX slots and READBACK_BINS bins.
+// positions of 2048 particles (2624 slots) to the host: 221 us that way, 45 us
+// so; of 6144 (7936 slots) 213 and 68 us.
+// For up to READBACK_MAX slots and READBACK_BINS bins.  The work grows with the
+// square of the particles, but the two meet only at about 45000 slots (20992: 217
+// and 127 us, 41472: 242 and 225, 82944: 267 and 523): READBACK_MAX is well on
+// the safe side.
 constexpr int RB_STAGE = 2048;
 
 __global__ void __launch_bounds__(WG)
