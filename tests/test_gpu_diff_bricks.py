@@ -1,9 +1,11 @@
 """The differentiable box's particle phase by bricks, at the sizes where its
 layout changes: sides shorter than a brick, ragged sides, bricks of 4 and of 8
 cells, every length of a particle block, boxes whose bricks take their particles
-through a list, moves longer than a cell, and particles outside the box.  FP64 against the
-PyTorch PIC and its autograd (bars of test_gpu_diff.py: 1e-12 forward, 1e-9
-adjoint)."""
+through a list or are split over workgroups, moves longer than a cell, and
+particles outside the box.  FP64 against the PyTorch PIC and its autograd (bars of
+test_gpu_diff.py: 1e-12 forward, 1e-9 adjoint; FP32 boxes in these layouts:
+test_gpu_ensemble.py).  Where a layout once made boxes of some shape slow, their
+time is held against a like box that it suits."""
 
 import numpy as np
 import pytest
